@@ -67,6 +67,11 @@ def _log(rng, lo, hi):
     return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
 
 
+def _width(rng):
+    """An input width that the projections take: up to 2048 or 3136 to 6144, a multiple of 64."""
+    return 64 * (_log(rng, 8, 32) if rng.random() < 0.5 else _log(rng, 49, 96))
+
+
 def draw(rng):
     kind = rng.choice(["proj", "mlp", "gdn", "attn", "head", "gemm", "gemm", "load", "attn", "prefill", "request"])
     if kind == "proj":
@@ -74,12 +79,12 @@ def draw(rng):
             rows, K = rng.choice([(5120, 17408), (16384, 5120), (10240, 5120), (14336, 5120), (5120, 6144),
                                   (5120, 4096), (34816, 5120), (4096, 1024), (1024, 2048)])
         else:
-            rows, K = _log(rng, 256, 34816), 64 * _log(rng, 8, 272)
+            rows, K = _log(rng, 256, 34816), _width(rng)
         return {"kind": kind, "rows": rows, "K": K, "nr": rng.randint(1, 8), "bf16": rng.random() < 0.5,
                 "res": rng.choice(["none", "bf16", "f32"])}
     if kind == "mlp":
-        hidden = 1024 * rng.randint(1, 5)
-        return {"kind": kind, "hidden": hidden, "inter": 64 * _log(rng, 16, 272), "nr": rng.randint(1, 8)}
+        return {"kind": kind, "hidden": 1024 * rng.choice([1, 2, 4, 5]), "inter": rng.choice([INTER, 2048, _width(rng)]),
+                "nr": rng.randint(1, 8)}
     if kind == "gdn":
         kh = rng.choice([1, 2, 4, 8, 16])
         nr = rng.randint(1, 8)
