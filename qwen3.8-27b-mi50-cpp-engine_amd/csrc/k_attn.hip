@@ -594,21 +594,44 @@ __global__ __launch_bounds__(HD) void k_attn_combine(AttnArgs a, int nr) {
 // V from the cache. The splits, and the order of every sum, are those of the kernels above and of
 // the oracle: score = ((c0 + c1) + c2) + c3 with c_j the fmaf chain over dims [j HD/4, (j+1) HD/4),
 // on K values code x scale; the split softmax m = max, p = 2^(x - m), l = the 64-lane shfl_down
-// tree; o = ((o0 + o1) + o2) + o3 with o_j the fmaf chain over the row's visible keys of the split's
-// j-th 16-key block, in key order. Block = (split, kv head), all rows and GQA heads of the kv head:
-// the int8 K/V tile and its scales in LDS (an fp32 tile of 256-wide rows would not leave room for
-// the queries), plain VALU chains, one thread per (query, key) score and per (query, dim) output.
+// tree; o = ((o0 + o1) + o2) + o3 with o_j the fmaf chain over the split's j-th 16-key block in key
+// order (keys a row does not see have p = 0).
+//
+// Block = (split, kv head), all rows and GQA heads of the kv head as QT tiles of 16 query vectors,
+// 8 waves, on v_mfma_f32_16x16x4f32 (an instruction adds its four products one after another with
+// fused multiply-adds, so a chain of them is an fmaf loop). Bound by the fp32 matrix rate (157
+// TFLOP/s): the int8 K/V bytes are a third of that time at 48 query vectors.
+//   K/V: int8 tiles and their scales by LDS DMA, one split ahead in a second buffer, 16-byte chunk
+//     c of key row R in slot c ^ (R % (HD/16)), so the 16 keys of an operand read hit distinct
+//     banks; codes are widened and scaled as operands are read (an fp32 tile of 256-wide rows
+//     would not leave room, and costs a pass and a barrier of its own).
+//   scores: wave (key tile kt, half h) runs chains 2h and 2h + 1 (its half of the dims) of all QT
+//     query tiles, the queries in registers for the whole launch; every wave has the same work at
+//     any QT. c0 + c1, c2 and c3 meet in LDS, where the softmax adds them.
+//   P.V: wave w owns HD/128 16-dim tiles for all query tiles.
 constexpr int kGThreads = 512;
-constexpr int kSpG = kSplit + 1;                 // score row stride (floats)
+// x, as a value the compiler cannot move out of the loop it is taken in
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+constexpr int kSpG = kSplit + 4;                 // score row stride (floats)
+// Dynamic LDS of a launch with QT query tiles: 2 x (K, V codes) | 2 x (K, V scales) | 3 score arrays
+// (the query stage before the first scores)
 template <int HD>
-__host__ __device__ constexpr int tile_stride_g() { return HD + 16; }   // int8 K/V tile row stride
-template <int HD>
+__host__ __device__ constexpr size_t split_g_lds(int qt) {
+    return (size_t)4 * kSplit * HD + (size_t)4 * kSplit * (HD / 16) * 4 + (size_t)3 * qt * 16 * kSpG * 4;
+}
+template <int HD, int QT>
 __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) {
+    warm_args(a);
     if (stopped(a.stop)) return;
-    constexpr int KS = tile_stride_g<HD>();
-    constexpr int NSC = HD / 16;                 // scales per key row at most (kv_group >= 16)
+    constexpr int NCH = HD / 16;                 // 16-byte chunks per key row; scales per row at most
+    constexpr int NS = HD / 8;                   // K elements of a lane: its half's dims 4 s + g
+    constexpr int NQ = 16 * QT;
     const int kvh = blockIdx.y;
     const int G = a.nq / a.nkv;
+    const uint32_t gdiv = (65536u + G - 1) / G;     // i / G = i gdiv >> 16 for i < 64
     int nact = a.nact_ptr ? ld_uniform(a.nact_ptr) : nr;
     int pos0 = a.pos0_ptr ? ld_uniform(a.pos0_ptr) : a.pos0_imm;
     if (a.zrows) tile_rows<HD>(a, nr, pos0, nact);
@@ -616,94 +639,252 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
     const int nqr = nact * G;
     const int kvrows = a.nkv * HD;
     const int ms = a.max_splits;
-    const int KG = a.kv_group, nsc = HD / KG;
-    __shared__ __attribute__((aligned(16))) int8_t k8[kSplit * KS];
-    __shared__ __attribute__((aligned(16))) int8_t v8[kSplit * KS];
-    __shared__ float ksc[kSplit * NSC];
-    __shared__ float vsc[kSplit * NSC];
-    extern __shared__ float dyn[];
-    float* qf = dyn;                                // [nr G][HD] queries as fp32
-    float* sp = dyn + (size_t)nr * G * HD;          // [nr G][kSpG] scores, then p
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int gsh = __builtin_ctz(a.kv_group), nsc = HD >> gsh;     // kv_group is 16, 32 or 64
+    extern __shared__ __attribute__((aligned(16))) int8_t gdyn[];
+    int8_t* kv8 = gdyn;                                             // [2][K | V][64][HD]
+    float* scl = (float*)(gdyn + 4 * kSplit * HD);                  // [2][K | V][64][nsc] (room for NCH)
+    float* sp = scl + 4 * kSplit * NCH;                             // [NQ][kSpG] c0 + c1, then p
+    float* sc2 = sp + NQ * kSpG;                                    // c2
+    float* sc3 = sc2 + NQ * kSpG;                                   // c3
+    __shared__ int sbad[2];                                         // per buffer: a hidden V row is not finite
+    const int t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int g4 = lane >> 4, j16 = lane & 15;
     float* wo = a.work;
     float* wm = a.work + (size_t)nr * a.nq * ms * HD;
     float* wl = wm + (size_t)nr * a.nq * ms;
-    for (int i = t; i < nqr * HD; i += kGThreads) {
-        const int qi = i / HD, d = i - qi * HD;
-        const int r = qi / G, g = qi - r * G;
-        qf[i] = bf2f(a.qh[(size_t)r * a.nq * HD + (size_t)(kvh * G + g) * HD + d]);
+    int s = blockIdx.x;
+    if (s * kSplit >= Lmax) return;
+    // split s into buffer b: 1 KiB of codes per wave instruction (64 / NCH key rows), then one scale
+    // per lane; keys past the last read the split's first key (visible to every row that uses the
+    // split, so it adds nothing that is not there already)
+    const uint32_t kv_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)kv8;
+    const uint32_t scl_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)scl;
+    auto load_tile = [&](int sn, int b) __attribute__((always_inline)) {
+        const int k0 = sn * kSplit;
+        const int nk = (Lmax - k0 < kSplit) ? (Lmax - k0) : kSplit;
+        constexpr int RPI = 64 / NCH, NI = kSplit / RPI;            // rows per instruction, instructions per matrix
+        const int lane = opaque((int)threadIdx.x & 63);
+#pragma unroll
+        for (int i = 0; i < 2 * NI / 8; ++i) {
+            const int u = wv + 8 * i, isv = u / NI, R = (u % NI) * RPI + lane / NCH;
+            const int c = (lane % NCH) ^ (R % NCH);
+            const size_t off = (size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD + 16 * c;
+            lds_dma16((isv ? a.vc : a.kc) + off,
+                      __builtin_amdgcn_readfirstlane(kv_lds + (uint32_t)((2 * b + isv) * kSplit * HD + 1024 * (u % NI))));
+        }
+        for (int u = wv; u < 2 * nsc; u += 8) {                     // nsc instructions of 64 scales per matrix
+            const int isv = u >= nsc, i = isv ? u - nsc : u;
+            const int f = 64 * i + lane, R = f >> (__builtin_ctz(HD) - gsh), c = f & (nsc - 1);
+            const size_t off = (((size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD) >> gsh) + c;
+            lds_dma4((isv ? a.vs : a.ks) + off,
+                     __builtin_amdgcn_readfirstlane(scl_lds + (uint32_t)((2 * b + isv) * kSplit * NCH + 64 * i) * 4u));
+        }
+    };
+    load_tile(s, 0);
+    // queries: bf16 rows to LDS with dims 8 c + g and 8 c + 4 + g paired in word [row][g][c], then each
+    // lane's values (query 16 qt + j16, dims HD/2 h + 4 s + g4) to registers
+    const int kt = wv & 3, h = wv >> 2;
+    float q[QT][NS];
+    {
+        constexpr int QS = HD / 2 + 4;                              // words per staged query row
+        uint32_t* sq = (uint32_t*)sp;
+        for (int i = t; i < NQ * (HD / 8); i += kGThreads) {
+            const int qi = i / (HD / 8), c = i % (HD / 8);
+            const int qc = qi < nqr ? qi : 0;                       // rows past nqr: computed, not stored
+            const int r = (int)((qc * gdiv) >> 16), g = qc - r * G;
+            const uint4 x = *(const uint4*)(a.qh + (size_t)r * a.nq * HD + (size_t)(kvh * G + g) * HD + 8 * c);
+            uint32_t* d = sq + qi * QS + c;
+            d[0] = __builtin_amdgcn_perm(x.z, x.x, 0x05040100u);
+            d[HD / 8] = __builtin_amdgcn_perm(x.z, x.x, 0x07060302u);
+            d[2 * (HD / 8)] = __builtin_amdgcn_perm(x.w, x.y, 0x05040100u);
+            d[3 * (HD / 8)] = __builtin_amdgcn_perm(x.w, x.y, 0x07060302u);
+        }
+        if (t == 0) sbad[0] = sbad[1] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+            for (int m = 0; m < NS / 8; ++m) {
+                const uint4 x = *(const uint4*)(sq + (16 * qt + j16) * QS + g4 * (HD / 8) + (NS / 2) * h + 4 * m);
+                const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    q[qt][8 * m + 2 * e] = __uint_as_float(w[e] << 16);
+                    q[qt][8 * m + 2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
+                }
+            }
     }
-    for (int s = blockIdx.x; s * kSplit < Lmax; s += gridDim.x) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));                       // this wave's transfers have landed
+    __syncthreads();                                                // every wave's; the query stage is read
+    for (int b = 0; s * kSplit < Lmax; s += gridDim.x, b ^= 1) {
         const int k0 = s * kSplit;
         const int nk = (Lmax - k0 < kSplit) ? (Lmax - k0) : kSplit;
-        __syncthreads();                            // the previous split's tiles are consumed
-        for (int i = t; i < nk * (HD / 16); i += kGThreads) {
-            const int k = i / (HD / 16), c = i - k * (HD / 16);
-            const size_t off = (size_t)(k0 + k) * kvrows + (size_t)kvh * HD + 16 * c;
-            *(uint4*)&k8[k * KS + 16 * c] = *(const uint4*)(a.kc + off);
-            *(uint4*)&v8[k * KS + 16 * c] = *(const uint4*)(a.vc + off);
+        const int8_t* k8 = kv8 + (size_t)(2 * b) * kSplit * HD;
+        const int8_t* v8 = k8 + kSplit * HD;
+        const float* ksc = scl + (2 * b) * kSplit * NCH;
+        const float* vsc = ksc + kSplit * NCH;
+        // the block's next split: in flight through this split's work
+        if ((s + (int)gridDim.x) * kSplit < Lmax) load_tile(s + gridDim.x, b ^ 1);
+        // A value that is not finite in a V row that some of the block's rows do not see (p = 0)
+        // would reach them through the matrix cores: such splits take P.V key by key.
+        if (k0 + nk > pos0 + 1) {
+            const int kf = pos0 + 1 > k0 ? pos0 + 1 - k0 : 0;       // first key that row 0 does not see
+            for (int i = kf * nsc + t; i < nk * nsc; i += kGThreads)
+                if (!(fabsf(vsc[i]) < __builtin_huge_valf())) sbad[b] = 1;
         }
-        for (int i = t; i < nk * nsc; i += kGThreads) {
-            const int k = i / nsc, c = i - k * nsc;
-            const size_t off = ((size_t)(k0 + k) * kvrows + (size_t)kvh * HD) / KG + c;
-            ksc[k * NSC + c] = a.ks[off];
-            vsc[k * NSC + c] = a.vs[off];
-        }
-        __syncthreads();
-        // scores, one (query, key) pair per thread at a time
-        for (int i = t; i < nqr * kSplit; i += kGThreads) {
-            const int qi = i >> 6, key = i & (kSplit - 1);
-            if (key >= nk) continue;
-            const float* q = qf + (size_t)qi * HD;
-            const int8_t* kr = k8 + key * KS;
-            const float* kscr = ksc + key * NSC;
-            float c4[4];
+        // (each phase takes the lane's indices anew: hoisted out of the loop, their addresses alone would
+        // not fit the registers beside the queries)
+        // ---- scores: lane 16 g + j supplies q(16 qt + j)[d] and k(16 kt + j)[d], d = HD/2 h + 4 s + g
+        {
+            const int ln = opaque(lane), g4 = ln >> 4, j16 = ln & 15;
+            const int key = 16 * kt + j16;
+            v4f acc[QT][2];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float acc = 0.0f;
-                for (int d = j * (HD / 4); d < (j + 1) * (HD / 4); ++d)
-                    acc = __builtin_fmaf(q[d], (float)kr[d] * kscr[d / KG], acc);
-                c4[j] = acc;
-            }
-            sp[(size_t)qi * kSpG + key] = (((c4[0] + c4[1]) + c4[2]) + c4[3]) * a.sl2e;
-        }
-        __syncthreads();
-        // split softmax, one wave per query, lane = key
-        for (int qi = wv; qi < nqr; qi += kGThreads / 64) {
-            const int r = qi / G, g = qi - r * G;
-            const int L = pos0 + r + 1;
-            const int nv = (L - k0 < nk) ? (L - k0) : nk;       // visible keys of this row in the split
-            const float x = (lane < nv) ? sp[(size_t)qi * kSpG + lane] : -__builtin_huge_valf();
-            const float m = max_xor(x, 64);
-            const float p = (lane < nv) ? qexp2(x - m) : 0.0f;
-            const float l = tree64(p);
-            sp[(size_t)qi * kSpG + lane] = p;
-            if (lane == 0 && nv > 0) {
-                const size_t mi = ((size_t)r * a.nq + (size_t)(kvh * G + g)) * ms + s;
-                wm[mi] = m;
-                wl[mi] = l;
-            }
-        }
-        __syncthreads();
-        // o = sum_k p_k v_k, one (query, dim) pair per thread at a time
-        for (int i = t; i < nqr * HD; i += kGThreads) {
-            const int qi = i / HD, d = i - qi * HD;
-            const int r = qi / G, g = qi - r * G;
-            const int L = pos0 + r + 1;
-            const int nv = (L - k0 < nk) ? (L - k0) : nk;
-            if (nv <= 0) continue;
-            const float* pr = sp + (size_t)qi * kSpG;
-            float o4[4];
+            for (int qt = 0; qt < QT; ++qt) acc[qt][0] = acc[qt][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float acc = 0.0f;
-                const int e = (16 * (j + 1) < nv) ? 16 * (j + 1) : nv;
-                for (int key = 16 * j; key < e; ++key)
-                    acc = __builtin_fmaf(pr[key], (float)v8[key * KS + d] * vsc[key * NSC + d / KG], acc);
-                o4[j] = acc;
+            for (int m = 0; m < NS / 8; ++m) {
+                // chunk m of each of the half's two chains
+                float k[2][4];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int ch = (NS / 4) * h + (NS / 8) * c + m;
+                    const uint4 x = *(const uint4*)(k8 + key * HD + ((ch ^ (key % NCH)) << 4));
+                    const float sc = ksc[key * nsc + ((16 * ch) >> gsh)];
+                    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) k[c][e] = (float)(int)(int8_t)(w[e] >> (8 * g4)) * sc;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+                            acc[qt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[qt][(NS / 2) * c + 4 * m + e], k[c][e],
+                                                                              acc[qt][c], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);   // (all chunks widened ahead do not fit the registers)
             }
-            wo[(((size_t)r * a.nq + (size_t)(kvh * G + g)) * ms + s) * HD + d] = ((o4[0] + o4[1]) + o4[2]) + o4[3];
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = (16 * qt + 4 * g4 + r) * kSpG + key;
+                    if (h == 0) {
+                        sp[i] = acc[qt][0][r] + acc[qt][1][r];
+                    } else {
+                        sc2[i] = acc[qt][0][r];
+                        sc3[i] = acc[qt][1][r];
+                    }
+                }
         }
+        __syncthreads();
+        if (t == 0) sbad[b ^ 1] = 0;                // (read in the split before, set at the earliest in the next)
+        // ---- split softmax as in k_attn_split: four queries of the wave at a time, lane 16 i + c holding
+        // keys c, c + 16, c + 32, c + 48 of the pass's i-th; p of key k goes to position
+        // 16 (k % 4) + k / 4 of the row, where a lane of P.V finds its 16 keys 4 s + g side by side
+#pragma unroll 1
+        for (int pass = 0; pass < (QT + 1) / 2; ++pass) {
+            const int ln = opaque(lane), g4 = ln >> 4, j16 = ln & 15;
+            const int qi = 32 * pass + 4 * wv + g4;
+            if (32 * pass + 4 * wv < nqr) {
+                const int qc = qi < nqr ? qi : nqr - 1;
+                const int r = (int)((qc * gdiv) >> 16), g = qc - r * G;
+                const int L = pos0 + r + 1;
+                const int nv = (L - k0 < nk) ? (L - k0) : nk;       // visible keys of this row in the split
+                float x[4], p[4];
+                float m = -__builtin_huge_valf();
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = qc * kSpG + j16 + 16 * e;
+                    x[e] = ((sp[i] + sc2[i]) + sc3[i]) * a.sl2e;
+                    if (j16 + 16 * e < nv) m = fmaxf(m, x[e]);
+                }
+                m = max_xor(m, 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[e] = (j16 + 16 * e < nv) ? qexp2(x[e] - m) : 0.0f;
+                float l = (p[0] + p[2]) + (p[1] + p[3]);
+                l = down_add<8>(l);
+                l = down_add<4>(l);
+                l = down_add<2>(l);
+                l = down_add<1>(l);
+                if (qi < nqr) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sp[qi * kSpG + 16 * (j16 & 3) + (j16 >> 2) + 4 * e] = p[e];
+                    if (j16 == 0 && nv > 0) {
+                        const size_t mi = ((size_t)r * a.nq + (size_t)(kvh * G + g)) * ms + s;
+                        wm[mi] = m;
+                        wl[mi] = l;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        const int bad = sbad[b];
+        // ---- o = sum_k p_k v_k: lane 16 g + j supplies p(16 qt + j)[4 s + g] and v(4 s + g)[16 dt + j]
+        // this wave's transfers of the next split have landed (waited for ahead of the stores below,
+        // which the count would include)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        float* ws = wo + ((size_t)(kvh * G) * ms + s) * HD;
+        auto put = [&](int qi, int d, float o) __attribute__((always_inline)) {
+            const int r = (int)((qi * gdiv) >> 16), g = qi - r * G;
+            if (pos0 + r + 1 - k0 > 0)             // some key of this split is visible to the row
+                ws[(uint32_t)((r * a.nq + g) * ms) * (uint32_t)HD + d] = o;
+        };
+        if (!bad) {
+#pragma unroll
+            for (int u = 0; u < HD / 128; ++u) {
+                const int ln = opaque(lane), g4 = ln >> 4, j16 = ln & 15;
+                const int dt = (HD / 128) * wv + u;
+                float v[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int key = 4 * e + g4;
+                    v[e] = (float)(int)v8[key * HD + ((dt ^ (key % NCH)) << 4) + j16] * vsc[key * nsc + ((16 * dt) >> gsh)];
+                }
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    const float4* pr = (const float4*)(sp + (16 * qt + j16) * kSpG + 16 * g4);
+                    v4f c[4];
+                    float4 p4[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) { c[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f}; p4[i] = pr[i]; }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(p4[i].x, v[4 * i], c[i], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(p4[i].y, v[4 * i + 1], c[i], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(p4[i].z, v[4 * i + 2], c[i], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(p4[i].w, v[4 * i + 3], c[i], 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int qi = 16 * qt + 4 * g4 + r;
+                        if (qi < nqr) put(qi, 16 * dt + j16, ((c[0][r] + c[1][r]) + c[2][r]) + c[3][r]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        } else {
+            for (int i = t; i < nqr * HD; i += kGThreads) {
+                const int qi = i / HD, d = i - qi * HD;
+                const int L = pos0 + (int)((qi * gdiv) >> 16) + 1;
+                const int nv = (L - k0 < nk) ? (L - k0) : nk;
+                float o4[4];
+                for (int j = 0; j < 4; ++j) {
+                    float acc = 0.0f;
+                    const int e = (16 * (j + 1) < nv) ? 16 * (j + 1) : nv;
+                    for (int key = 16 * j; key < e; ++key) {
+                        const int c = (d >> 4) ^ (key % NCH);
+                        acc = __builtin_fmaf(sp[qi * kSpG + 16 * (key & 3) + (key >> 2)],
+                                             (float)(int)v8[key * HD + (c << 4) + (d & 15)] * vsc[key * nsc + (d >> gsh)], acc);
+                    }
+                    o4[j] = acc;
+                }
+                put(qi, d, ((o4[0] + o4[1]) + o4[2]) + o4[3]);
+            }
+        }
+        __syncthreads();                            // the split is consumed, the next one landed
     }
 }
 
@@ -750,17 +931,25 @@ int launch_attn_prep_rows(const AttnArgs& a, int nrows, hipStream_t s) {
 
 template <int HD>
 static int launch_split_g(const AttnArgs& a, int nr, hipStream_t s) {
-    const size_t lds = (size_t)nr * (a.nq / a.nkv) * (HD + kSpG) * 4;
     static std::once_flag attr;
     static hipError_t attr_e = hipSuccess;
     std::call_once(attr, [] {
-        attr_e = hipFuncSetAttribute((const void*)k_attn_split_g<HD>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)((size_t)kMaxQ * (HD + kSpG) * 4));
+        const void* f[4] = {(const void*)k_attn_split_g<HD, 1>, (const void*)k_attn_split_g<HD, 2>,
+                            (const void*)k_attn_split_g<HD, 3>, (const void*)k_attn_split_g<HD, 4>};
+        for (int i = 0; i < 4 && attr_e == hipSuccess; ++i)
+            attr_e = hipFuncSetAttribute(f[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_g_lds<HD>(i + 1));
     });
     Q27X_HIP(attr_e);
+    const int qt = (nr * (a.nq / a.nkv) + 15) / 16;
     const int bx = a.max_splits < kSplitBlocks / a.nkv ? a.max_splits : (kSplitBlocks / a.nkv > 0 ? kSplitBlocks / a.nkv : 1);
     const dim3 grid(bx, a.nkv, a.zrows ? (unsigned)((a.ztotal + a.zrows - 1) / a.zrows) : 1u);
-    hipLaunchKernelGGL(k_attn_split_g<HD>, grid, dim3(kGThreads), lds, s, a, nr);
+    const size_t lds = split_g_lds<HD>(qt);
+    switch (qt) {
+        case 1: hipLaunchKernelGGL((k_attn_split_g<HD, 1>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        case 2: hipLaunchKernelGGL((k_attn_split_g<HD, 2>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        case 3: hipLaunchKernelGGL((k_attn_split_g<HD, 3>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        default: hipLaunchKernelGGL((k_attn_split_g<HD, 4>), grid, dim3(kGThreads), lds, s, a, nr); break;
+    }
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }

@@ -110,6 +110,14 @@ __device__ __forceinline__ void lds_dma16(const void* g, uint32_t lds) {
                  : "=&s"(save) : "s"(lds), "v"(g) : "memory");
 }
 
+// The same for 4 bytes per lane: lane l's word from g lands at LDS byte address lds + 4 l.
+__device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
+    uint32_t save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+                 "global_load_lds_dword %2, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(save) : "s"(lds), "v"(g) : "memory");
+}
+
 // The round's stop flag (null: never stopped), read through the constant address space so it is
 // a scalar load: a vector load would make the wait for it (vmcnt) also wait for every weight load
 // issued before it. The flag does not change while a kernel that reads it runs.

@@ -363,6 +363,46 @@ def test_attention_group_6_at_128(gpu, O):
     attention_case(gpu, O, 700, 24, 4, 128, 32, 32, 3, 0x51E70021)
 
 
+@pytest.mark.parametrize("nq,nkv,hd,group,nr,L0,bad", [
+    (24, 4, 256, 16, 2, 62, False),        # one query tile, rows straddling a split, 16 scales per key
+    (24, 4, 256, 64, 4, 128, False),       # two tiles, a split that starts with the first new row
+    (24, 4, 256, 32, 8, 4500, False),      # three full tiles, two splits per block
+    (16, 2, 256, 32, 8, 63, False),        # four tiles (GQA group 8)
+    (7, 1, 128, 16, 1, 0, False),          # one key
+    (15, 3, 128, 64, 5, 190, False),       # two tiles (group 5)
+    (6, 2, 128, 32, 8, 9000, False),       # two tiles (group 3), two splits per block
+    (7, 1, 128, 32, 7, 500, False),        # four tiles, 49 of 64 rows
+    (24, 4, 256, 32, 3, 61, True), (24, 4, 256, 32, 3, 62, True), (6, 2, 128, 32, 3, 125, True)])
+def test_attention_general_tiles(gpu, O, nq, nkv, hd, group, nr, L0, bad):
+    """The general attention kernel at the edges of its query tiles, splits and scale groups, on a
+    cache that holds every position; bad: the last position's V scales are infinite, which only the
+    last row may see (the earlier rows' weights on that key are zero)."""
+    X = gpu
+    rng = np.random.default_rng(L0 + 100 * nr + hd)
+    ctx = L0 + nr
+    kc, ks, vc, vs = fill_kv(rng, O, ctx, nkv, hd, group, ctx)
+    if bad:
+        vs[ctx - 1] = np.inf
+    qh = bf16_normal(rng, (nr, nq * hd), 1.0, O=O)
+    gates = bf16_normal(rng, (nr, 2 * nq * hd), 1.0, O=O)
+    out_o = np.empty((nr, nq * hd), np.uint16)
+    xq_o, xs_o = np.empty((nr, nq * hd), np.int8), np.empty((nr, nq * hd // 16), np.float32)
+    O.lib().q27o_attn_rows(qh.ctypes.data, gates.ctypes.data, 2 * nq * hd, kc.ctypes.data, ks.ctypes.data, vc.ctypes.data,
+                           vs.ctypes.data, group, nq, nkv, hd, 1, L0, nr, out_o.ctypes.data, xq_o.ctypes.data,
+                           xs_o.ctypes.data)
+    dq, dg, dk, dks, dv, dvs = dev(X, qh), dev(X, gates), dev(X, kc), dev(X, ks), dev(X, vc), dev(X, vs)
+    work = X.DevBuf(X.lib().q27x_attn_work_bytes(nq, hd, ctx, nr))
+    dout, dxq, dxs = X.DevBuf(nr * nq * hd * 2), X.DevBuf(nr * nq * hd), X.DevBuf(nr * nq * hd // 4)
+    X.call("q27x_attn_rows", dq.ptr, dg.ptr, 2 * nq * hd, dk.ptr, dks.ptr, dv.ptr, dvs.ptr, group, nq, nkv, hd, 1, L0, nr,
+           work.ptr, dout.ptr, dxq.ptr, dxs.ptr, None)
+    X.call("q27x_device_sync")
+    rows = nr - 1 if bad else nr
+    same("attention out", dout.download(np.uint16, (nr, nq * hd))[:rows], out_o[:rows])
+    same("attention codes", dxq.download(np.int8, (nr, nq * hd))[:rows], xq_o[:rows])
+    same("attention scales", dxs.download(np.float32, (nr, nq * hd // 16))[:rows], xs_o[:rows])
+    assert np.isfinite(xs_o[:rows]).all()
+
+
 def test_accept(gpu):
     X = gpu
     for nx, dt, exp in (([5, 6, 7], [5, 6], 2), ([5, 6, 7], [5, 9], 1), ([5, 6, 7], [4, 6], 0), ([1], [], 0)):
