@@ -17,17 +17,16 @@
 // The int32 group sums do not depend on the order of their terms, so the MFMA tiling cannot
 // change them; the fp32 part runs per output in the reference's group order.
 //
-// GEMM tiling: a 256-thread block computes a 128-token x 128-row tile; wave w owns the 64 x 64
-// quarter (w / 2, w % 2) as 2 x 2 v_mfma_i32_32x32x32_i8 tiles, and two blocks share a CU. K
-// advances 64 bytes per stage through a ring of 4 LDS stages (3 when the scales of 17+ groups
-// take the room) filled by LDS DMA ahead of the multiply, so 96-128 KiB per CU stay in flight
-// to cover the memory latency (one stage ahead measured 16% of the int8 peak: every stage waited
-// for its own loads). At the end of each group the int32 tiles are folded into fp32
-// accumulators with the group's scales (staged in LDS for the whole K at the start) and
-// restarted from zero. Larger forms: 256-token tiles (k_gemm_i8g_rs, 8 waves), and with one group
-// over the whole K 256 x 256 tiles (k_gemm_i8g_w4, 8 waves of 128 x 64) where the launch needs
-// fewer tile rounds with them.
+// GEMM tiling: a launch takes the cheapest of a list of forms (launch_gemm_i8g): k_gemm_i8g_ring (64 to 256 tokens
+// x 64 to 256 weight rows per block, 128-byte K stages in an LDS ring), k_gemm_i8g_sk (few tokens: small tiles whose
+// waves split K), k_gemm_i8g_w4 (256 x 256 tiles, one group over K) and k_gemm_i8g_rs (256 x 128, many groups). At
+// the end of each group the int32 tiles are folded into fp32 accumulators with the group's scales and restarted
+// from zero. The general form for the other shapes, k_gemm_i8g: a 256-thread block computes a 128-token x 128-row
+// tile; wave w owns the 64 x 64 quarter (w / 2, w % 2) as 2 x 2 v_mfma_i32_32x32x32_i8 tiles, and two blocks share a
+// CU. K advances 64 bytes per stage through a ring of 4 LDS stages (3 when the scales of 17+ groups take the room)
+// filled by LDS DMA ahead of the multiply.
 #include <stdlib.h>
+#include <mutex>
 #include <type_traits>
 
 #include "q27x_dev.h"
@@ -39,6 +38,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kGN = 128, kGK = 64;                // block tile: BM tokens x 128 weight rows, 64 K bytes per stage
+constexpr int kSkLds = 160 * 1024;                 // LDS of the split-K kernel
 constexpr int kGMaxG = 20;                         // groups per row held in LDS (K / GS)
 template <int BM, int NS> struct GemmCfg {
     static constexpr int S = NS;                   // stages in the LDS ring
@@ -531,6 +531,340 @@ __global__ __launch_bounds__(512) void k_gemm_i8g_w4(GemmArgs a) {
     else out(std::false_type{});
 }
 
+// 128-byte stages (a stage row is one whole 128-byte line of a row) through a ring of S LDS stages filled by LDS
+// DMA: 64 WM tokens x 64 WN weight rows per block, each wave 64 x 64 as 2 x 2 v_mfma_i32_32x32x32_i8 tiles; with
+// KS = 2 two waves share a 64 x 64 quarter, each multiplying two of the stage's four 32-byte slices (their sums meet
+// in LDS at the end). Operand reads run one slice ahead of the MFMAs, across the stage barrier too, as in
+// k_gemm_i8g_w4. Same tile order and row swizzle.
+template <int WM, int WN, int KS, int S> struct RingCfg {
+    static constexpr int BM = 64 * WM, BN = 64 * WN, NW = WM * WN * KS;
+    static constexpr int Stage = (BM + BN) * 128, NI = Stage / (1024 * NW);
+    static constexpr int Ring = S * Stage;
+    static_assert(Stage % (1024 * NW) == 0 && NI * (S - 1) < 64, "whole transfers per wave");
+};
+template <int WM, int WN, int KS, int S, bool GRP>
+__global__ __launch_bounds__(64 * WM * WN * KS) void k_gemm_i8g_ring(GemmArgs a) {
+    using C = RingCfg<WM, WN, KS, S>;
+    static_assert(!GRP || KS == 1, "group sums are folded by one wave");
+    constexpr int BM = C::BM, BN = C::BN, NT = 64 * C::NW, NI = C::NI, SL = 4 / KS;
+    extern __shared__ __attribute__((aligned(16))) int8_t rgdyn[];     // [S][Stage] | scales [BM][ng] | [BN][ng]
+    float* sSx = (float*)(rgdyn + C::Ring);
+    float* sSw = sSx + BM * a.ng;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
+    const int nt = a.N / BN, mt = (a.M + BM - 1) / BM, T = nt * mt;
+    const int b = blockIdx.x, xq = T / 8, xr = T % 8, xi = b % 8;
+    const int tile = xi * xq + (xi < xr ? xi : xr) + b / 8;
+    const int grp = tile / (4 * nt), fm = grp * 4, gsz = (mt - fm < 4) ? mt - fm : 4;
+    const int within = tile - grp * 4 * nt;
+    const int m0 = (fm + within % gsz) * BM, n0 = (within / gsz) * BN;
+    const int K = a.K, ng = a.ng, nst = K / 128, spg = a.gs / 128;
+    uint32_t off[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int rs = 8 * (NI * wave + i) + (lane >> 3), r = rs < BM ? rs : rs - BM;
+        const int c = (lane & 7) ^ ((r >> 1) & 7);
+        off[i] = (uint32_t)(rs >= BM ? n0 + r : m0 + r < a.M ? m0 + r : a.M - 1) * (uint32_t)K + 16u * c;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)rgdyn + 1024 * NI * wave;
+    auto issue = [&](int st, int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+            lds_dma16_at((8 * (NI * wave + i) < BM ? a.x : a.w) + (size_t)st * 128, off[i],
+                         __builtin_amdgcn_readfirstlane(lds0 + slot * C::Stage + 1024 * i));
+    };
+#pragma unroll
+    for (int p = 0; p < S; ++p) issue(p < nst ? p : 0, p);
+    for (int i = tid; i < BM * ng; i += NT) {
+        const int r = i / ng, t = m0 + r < a.M ? m0 + r : a.M - 1;
+        sSx[i] = a.sx[(size_t)t * ng + (i - r * ng)];
+    }
+    for (int i = tid; i < BN * ng; i += NT) sSw[i] = a.sw[(size_t)n0 * ng + i];
+    v16i acc[2][2];
+    float facc[GRP ? 2 : 1][GRP ? 2 : 1][GRP ? 16 : 1];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = 0;
+                if constexpr (GRP) facc[i][j][r] = 0.0f;
+            }
+    const int arow = wm * 64 + (lane & 31), brow = wn * 64 + (lane & 31);
+    const int swa = (arow >> 1) & 7, swb = (brow >> 1) & 7, kh = lane >> 5;
+    auto rd = [&](v4i (&av)[2], v4i (&bv)[2], int slot, int kk) __attribute__((always_inline)) {
+        const int8_t* st = rgdyn + slot * C::Stage;
+        const int c = 2 * (SL * kg + kk) + kh;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) av[i] = *(const v4i*)(st + (arow + 32 * i) * 128 + ((c ^ swa) << 4));
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bv[j] = *(const v4i*)(st + (BM + brow + 32 * j) * 128 + ((c ^ swb) << 4));
+    };
+    // at most `left` stages' transfers of this wave outstanding and its operand reads returned, then the barrier
+    auto sync = [&](auto left) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(NI * decltype(left)::value) & ~(15 << 8));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    v4i oa[2][2], ob[2][2];
+    sync(std::integral_constant<int, S - 1>{});
+    rd(oa[0], ob[0], 0, 0);
+    int slot = 0, gl = spg, g = 0;
+    for (int s = 0; s < nst; ++s) {
+        const int sn = slot + 1 == S ? 0 : slot + 1;
+#pragma unroll
+        for (int kk = 0; kk < SL; ++kk) {
+            const int cu = kk & 1, nx = cu ^ 1;
+            if (kk + 1 < SL) {
+                rd(oa[nx], ob[nx], slot, kk + 1);
+            } else {
+                // stage s + 1 landed everywhere and stage s is read by all: its slot takes stage s + S (past the
+                // end: stage 0 again, so every iteration issues the same transfers)
+                sync(std::integral_constant<int, S - 2>{});
+                issue(s + S < nst ? s + S : 0, slot);
+                rd(oa[nx], ob[nx], sn, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(oa[cu][i], ob[cu][j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        }
+        slot = sn;
+        if constexpr (GRP) {
+            if (--gl == 0) {
+                gl = spg;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float swv = sSw[(brow + 32 * j) * ng + g];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int tr = wm * 64 + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                            facc[i][j][r] = __builtin_fmaf((float)acc[i][j][r], swv * sSx[tr * ng + g], facc[i][j][r]);
+                            acc[i][j][r] = 0;
+                        }
+                }
+                ++g;
+            }
+        }
+    }
+    // no transfer may still be writing LDS when the block ends
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    if constexpr (KS == 2) {
+        // the two slice halves of a quarter: each wave gives the other its sums of the other's token half
+        __syncthreads();
+        int* ex = (int*)rgdyn + (wave % (WM * WN)) * 2 * 32 * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ex[((kg ^ 1) * 32 + j * 16 + r) * 64] = kg ? acc[0][j][r] : acc[1][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][j][r] = (kg ? acc[1][j][r] : acc[0][j][r]) + ex[(kg * 32 + j * 16 + r) * 64];
+    }
+    const uint32_t nb = (uint32_t)(n0 + wn * 64 + (lane & 31));
+    float swv[2], al[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        swv[j] = GRP ? 0.0f : sSw[wn * 64 + 32 * j + (lane & 31)];
+        al[j] = alpha_of(a.alpha, a.asel, (int)nb + 32 * j);
+    }
+    auto out = [&](auto res, auto obf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2 / KS; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int tl = wm * 64 + 32 * (KS == 2 ? kg : i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), t = m0 + tl;
+                if (t < a.M) {
+                    const uint32_t yo = (uint32_t)t * (uint32_t)a.ldy + nb, ro = (uint32_t)t * (uint32_t)a.ldr + nb;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        float o;
+                        if constexpr (GRP) o = facc[i][j][r] * al[j];
+                        else o = __builtin_fmaf((float)acc[i][j][r], swv[j] * sSx[tl], 0.0f) * al[j];
+                        if constexpr (decltype(res)::value == 1) o = o + a.rs * a.res[ro + 32 * j];
+                        if constexpr (decltype(res)::value == 2) o = o + a.rs * bf2f(((const uint16_t*)a.res)[ro + 32 * j]);
+                        if constexpr (decltype(obf)::value) ((uint16_t*)a.y)[yo + 32 * j] = f2bf(o);
+                        else a.y[yo + 32 * j] = o;
+                    }
+                }
+            }
+    };
+    auto form = [&](auto res) __attribute__((always_inline)) {
+        if (a.out_bf16) out(res, std::true_type{});
+        else out(res, std::false_type{});
+    };
+    if (!a.res) form(std::integral_constant<int, 0>{});
+    else if (a.res_bf16) form(std::integral_constant<int, 2>{});
+    else form(std::integral_constant<int, 1>{});
+}
+
+// Few tokens, or few weight rows for the CUs: a block of NW waves owns 16 RT weight rows x 16 MT tokens and its
+// waves split K, so every wave keeps the whole tile in registers (RT x MT v_mfma_i32_16x16x64_i8 tiles) and moves
+// its own operands through its own LDS ring (S stages of 128 K bytes, LDS DMA): the main loop has no barrier. The
+// waves' int32 sums are exact in any order: they meet in LDS (ds_add) in one slot per group, then every thread
+// folds its outputs in group order. gpp groups fit the slots at a time; more groups take further phases, whose
+// transfers are already in flight.
+template <int RT, int MT, int NW, int S> struct SkCfg {
+    static constexpr int Rows = 16 * (RT + MT), Stage = Rows * 128, NI = Rows / 8;    // 1 KiB transfers per stage
+    static constexpr int Ring = NW * S * Stage;
+    static constexpr int Out = 256 * RT * MT;          // outputs of the tile
+    static_assert(NI * (S - 1) < 64, "vector-memory count");
+};
+template <int RT, int MT, int NW, int S>
+__global__ __launch_bounds__(64 * NW) void k_gemm_i8g_sk(GemmArgs a, int gpp) {
+    using C = SkCfg<RT, MT, NW, S>;
+    constexpr int NT = 64 * NW, NO = C::Out, NPT = (NO + NT - 1) / NT, NI = C::NI;
+    // rings [NW][S][Stage] | [gpp][NO] int32 | token scales [16 MT][ng] | row scales [16 RT][ng]
+    extern __shared__ __attribute__((aligned(16))) int8_t skdyn[];
+    const int ng = a.ng, K = a.K;
+    int* sAcc = (int*)(skdyn + C::Ring);
+    float* sSx = (float*)(sAcc + (size_t)gpp * NO);
+    float* sSw = sSx + 16 * MT * ng;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // tiles with the token tile fastest, in one contiguous run per XCD (blocks go to the XCDs round-robin), so the
+    // blocks that share weight rows share an L2
+    const int mt = (a.M + 16 * MT - 1) / (16 * MT), T = gridDim.x, b = blockIdx.x;
+    const int xq = T / 8, xr = T % 8, xi = b % 8;
+    const int tile = xi * xq + (xi < xr ? xi : xr) + b / 8;
+    const int m0 = (tile % mt) * 16 * MT, n0 = (tile / mt) * 16 * RT;
+    // transfer i fills stage rows 8 i .. 8 i + 7 (weight rows, then tokens): lane l row 8 i + l / 8, slot l % 8, which
+    // holds chunk (l % 8) ^ ((row >> 1) & 7) of the row's 128 bytes (rows past M repeat row M - 1)
+    uint32_t off[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int row = 8 * i + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        const int t = m0 + row - 16 * RT;
+        off[i] = (uint32_t)(i < 2 * RT ? n0 + row : t < a.M ? t : a.M - 1) * (uint32_t)K + 16u * c;
+    }
+    const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)skdyn + wave * S * C::Stage;
+    auto issue = [&](int st, int slot) __attribute__((always_inline)) {
+        const int8_t* px = a.x + (size_t)st * 128;
+        const int8_t* pw = a.w + (size_t)st * 128;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+            lds_dma16_at(i < 2 * RT ? pw : px, off[i], __builtin_amdgcn_readfirstlane(ring + slot * C::Stage + 1024 * i));
+    };
+    const int nst = K / 128, spg = a.gs / 128, spp = spg * gpp;      // stages: all, per group, per phase
+    // this wave's stages of the phase that starts at stage p0
+    auto range = [&](int p0, int& s0, int& s1) __attribute__((always_inline)) {
+        const int pn = nst - p0 < spp ? nst - p0 : spp;
+        s0 = p0 + pn * wave / NW;
+        s1 = p0 + pn * (wave + 1) / NW;
+    };
+    // the stage to issue next: the wave's ranges one after another (past the last: stage 0 again, so every iteration
+    // issues the same transfers and the count stays exact)
+    int ip = 0, is = 0, ie = 0;
+    range(0, is, ie);
+    auto next = [&]() __attribute__((always_inline)) {
+        while (is >= ie && ip + spp < nst) { ip += spp; range(ip, is, ie); }
+        return is < ie ? is++ : 0;
+    };
+#pragma unroll
+    for (int p = 0; p < S - 1; ++p) issue(next(), p);
+    for (int i = tid; i < 16 * MT * ng; i += NT) {
+        const int r = i / ng, t = m0 + r < a.M ? m0 + r : a.M - 1;
+        sSx[i] = a.sx[(size_t)t * ng + (i - r * ng)];
+    }
+    for (int i = tid; i < 16 * RT * ng; i += NT) sSw[i] = a.sw[(size_t)n0 * ng + i];
+    for (int i = tid; i < gpp * NO; i += NT) sAcc[i] = 0;
+    __syncthreads();
+    v4i acc[RT][MT];
+    float o[NPT];
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) o[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = v4i{0, 0, 0, 0};
+    const int sw = (lane & 15) >> 1;                   // ((row >> 1) & 7) of this lane's operand rows
+    int slot = 0;
+    for (int p0 = 0, g0 = 0; p0 < nst; p0 += spp, g0 += gpp) {
+        const int gn = (nst - p0 < spp ? nst - p0 : spp) / spg;
+        int s0, s1;
+        range(p0, s0, s1);
+        int left = spg - s0 % spg, as = s0 / spg - g0;               // stages left of the current group, its slot
+        for (int s = s0; s < s1; ++s) {
+            // the slot read in the iteration before takes the stage S - 1 ahead; this stage has landed once at
+            // most the S - 1 stages behind it are outstanding (vector-memory counts retire in order)
+            issue(next(), slot == 0 ? S - 1 : slot - 1);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(NI * (S - 1)));
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            __builtin_amdgcn_sched_barrier(0);
+            const int8_t* st = skdyn + (wave * S + slot) * C::Stage + (lane & 15) * 128;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                const int c = ((4 * kk + (lane >> 4)) ^ sw) << 4;
+                v4i wv[RT], xv[MT];
+#pragma unroll
+                for (int j = 0; j < RT; ++j) wv[j] = *(const v4i*)(st + 16 * j * 128 + c);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) xv[i] = *(const v4i*)(st + 16 * (RT + i) * 128 + c);
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < RT; ++j)
+                        acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv[i], wv[j], acc[j][i], 0, 0, 0);
+            }
+            slot = slot + 1 == S ? 0 : slot + 1;
+            if (--left == 0 || s + 1 == s1) {
+#pragma unroll
+                for (int j = 0; j < RT; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            __hip_atomic_fetch_add(&sAcc[as * NO + ((j * MT + i) * 4 + r) * 64 + lane], acc[j][i][r],
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            acc[j][i][r] = 0;
+                        }
+                ++as;
+                left = spg;
+            }
+            // (the operand reads above have returned: their values are consumed before the slot is refilled)
+            __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0)
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        // output u: element r of lane's result in tile (j, i): token 16 i + 4 (lane / 16) + r, row 16 j + lane % 16
+#pragma unroll
+        for (int i = 0; i < NPT; ++i) {
+            const int u = tid + NT * i;
+            if (u < NO) {
+                const int tl = u >> 8, r = (u >> 6) & 3;
+                const float* px = sSx + (16 * (tl % MT) + 4 * (lane >> 4) + r) * ng + g0;
+                const float* pw = sSw + (16 * (tl / MT) + (lane & 15)) * ng + g0;
+                for (int g = 0; g < gn; ++g) {
+                    o[i] = __builtin_fmaf((float)sAcc[g * NO + u], pw[g] * px[g], o[i]);
+                    sAcc[g * NO + u] = 0;
+                }
+            }
+        }
+        if (p0 + spp < nst) __syncthreads();                        // the slots are read and cleared
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));          // no transfer may still be writing LDS when the block ends
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+        const int u = tid + NT * i, tl = u >> 8, r = (u >> 6) & 3;
+        const int t = m0 + 16 * (tl % MT) + 4 * (lane >> 4) + r, n = n0 + 16 * (tl / MT) + (lane & 15);
+        if (u < NO && t < a.M) {
+            float v = o[i] * alpha_of(a.alpha, a.asel, n);
+            if (a.res) v = v + a.rs * (a.res_bf16 ? bf2f(((const uint16_t*)a.res)[(size_t)t * a.ldr + n])
+                                                  : a.res[(size_t)t * a.ldr + n]);
+            if (a.out_bf16) ((uint16_t*)a.y)[(size_t)t * a.ldy + n] = f2bf(v);
+            else a.y[(size_t)t * a.ldy + n] = v;
+        }
+    }
+}
+
 // Weights: per-64 mirror -> per-(row, group) codes and scales; one 256-thread block per row.
 // In place when wg == w (each element is read and written by the same thread).
 __global__ __launch_bounds__(256) void k_i8g64_to_grp(const int8_t* w, const float* s64, int K, int gs,
@@ -639,6 +973,123 @@ static int gemm_cus() {
     }
     return g_gemm_cus;
 }
+template <int WM, int WN, int KS, int S, bool GRP>
+static int run_gemm_ring(const GemmArgs& a, hipStream_t s) {
+    using C = RingCfg<WM, WN, KS, S>;
+    const size_t lds = C::Ring + (size_t)(C::BM + C::BN) * a.ng * 4;
+    if (lds > kSkLds) { set_error("gemm: no LDS for %d groups", a.ng); return Q27X_E_SHAPE; }
+    static std::once_flag once;
+    static hipError_t e = hipSuccess;
+    std::call_once(once, [] {
+        e = hipFuncSetAttribute((const void*)k_gemm_i8g_ring<WM, WN, KS, S, GRP>, hipFuncAttributeMaxDynamicSharedMemorySize, kSkLds);
+    });
+    Q27X_HIP(e);
+    const unsigned grid = (unsigned)((a.N / C::BN) * ((a.M + C::BM - 1) / C::BM));
+    hipLaunchKernelGGL((k_gemm_i8g_ring<WM, WN, KS, S, GRP>), dim3(grid), dim3(64 * C::NW), lds, s, a);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+// the split-K kernel's launch: groups per phase by the LDS that their slots take beside the ring and the scales
+template <int RT, int MT, int NW, int S>
+static int run_gemm_sk(const GemmArgs& a, hipStream_t s) {
+    using C = SkCfg<RT, MT, NW, S>;
+    const size_t scl = (size_t)16 * (RT + MT) * a.ng * 4;
+    const int cap = ((int)kSkLds - C::Ring - (int)scl) / (C::Out * 4);
+    if (cap < 1) { set_error("gemm: no LDS for %d groups", a.ng); return Q27X_E_SHAPE; }
+    const int ph = (a.ng + cap - 1) / cap, gpp = (a.ng + ph - 1) / ph;
+    static std::once_flag once;
+    static hipError_t e = hipSuccess;
+    std::call_once(once, [] {
+        e = hipFuncSetAttribute((const void*)k_gemm_i8g_sk<RT, MT, NW, S>, hipFuncAttributeMaxDynamicSharedMemorySize, kSkLds);
+    });
+    Q27X_HIP(e);
+    const unsigned grid = (unsigned)((a.N / (16 * RT)) * ((a.M + 16 * MT - 1) / (16 * MT)));
+    hipLaunchKernelGGL((k_gemm_i8g_sk<RT, MT, NW, S>), dim3(grid), dim3(64 * NW), C::Ring + scl + (size_t)gpp * C::Out * 4, s, a, gpp);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+template <bool BF>
+static int run_gemm_w4(const GemmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)((a.N / kW4B) * ((a.M + kW4B - 1) / kW4B)));
+    if (!a.res) hipLaunchKernelGGL((k_gemm_i8g_w4<0, BF>), grid, dim3(512), 0, s, a);
+    else if (!a.res_bf16) hipLaunchKernelGGL((k_gemm_i8g_w4<1, BF>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((k_gemm_i8g_w4<2, BF>), grid, dim3(512), 0, s, a);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+template <bool BF>
+static int run_gemm_rs(const GemmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)((a.N / kGN) * ((a.M + 255) / 256)));
+    const size_t scl = (size_t)(256 + kGN) * a.ng * sizeof(float);
+    if (!a.res) hipLaunchKernelGGL((k_gemm_i8g_rs<0, BF>), grid, dim3(512), scl, s, a);
+    else if (!a.res_bf16) hipLaunchKernelGGL((k_gemm_i8g_rs<1, BF>), grid, dim3(512), scl, s, a);
+    else hipLaunchKernelGGL((k_gemm_i8g_rs<2, BF>), grid, dim3(512), scl, s, a);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+
+// The kernel forms and what a launch of each costs. A CU takes n = ceil(blocks / CUs) blocks, occ at a time; a block
+// runs K / 128 (/ ks) stages, t[r - 1] us per stage with r blocks on the CU; all blocks together read
+// (bm + bn) K bytes each at bw TB/s, and the weights come from HBM at 4.9 TB/s:
+//   us = a + max(stages (floor(n / occ) t[occ - 1] + t[n % occ - 1]), blocks (bm + bn) K / bw, N K / 4.9)
+// The constants are fits of measured launches (M = 1 .. 4096 at the model's nine widths, 216 shapes; per group of
+// 1024 columns 65 shapes). Over these the form taken is 3% off the fastest one on average. Before (128 x 128 tiles
+// of 64-byte stages below 512 tokens; from there 256 x 128 or 256 x 256) and now, us: M = 1, 5120 x 17408: 86 / 19;
+// M = 77: 102 / 33 (1024-column groups 125 / 45); M = 203, 5120 x 17408: 101 / 62, 34816 x 5120: 105 / 87;
+// M = 512: 129 / 82, 153 / 132; M = 1024, 5120 x 17408: 147 / 118; the 256 x 256 tiles stay for 1024 x 34816 up.
+enum { F_RING, F_SK, F_W4, F_RS };
+struct GemmForm {
+    int kind, bm, bn, ks, occ;
+    float a, t[3], bw;
+    int (*run)(const GemmArgs&, hipStream_t);
+};
+static int run_w4(const GemmArgs& a, hipStream_t s) { return a.out_bf16 ? run_gemm_w4<true>(a, s) : run_gemm_w4<false>(a, s); }
+static int run_rs(const GemmArgs& a, hipStream_t s) { return a.out_bf16 ? run_gemm_rs<true>(a, s) : run_gemm_rs<false>(a, s); }
+// one group over K
+static const GemmForm kFormsK[] = {
+    {F_SK, 16, 32, 4, 2, 3.57f, {0.316f, 0.653f}, 13.7f, run_gemm_sk<2, 1, 4, 3>},
+    {F_SK, 32, 32, 4, 2, 3.75f, {0.412f, 0.821f}, 16.0f, run_gemm_sk<2, 2, 4, 2>},
+    {F_SK, 32, 32, 2, 3, 4.19f, {0.337f, 0.450f, 0.505f}, 15.6f, run_gemm_sk<2, 2, 2, 2>},
+    {F_SK, 32, 64, 4, 1, 4.16f, {0.738f}, 13.7f, run_gemm_sk<4, 2, 4, 2>},
+    {F_SK, 64, 64, 4, 1, 6.34f, {0.983f}, 15.4f, run_gemm_sk<4, 4, 4, 2>},
+    {F_RING, 64, 64, 1, 3, 5.41f, {0.239f, 0.456f, 0.605f}, 15.2f, run_gemm_ring<1, 1, 2, 3, false>},
+    {F_RING, 64, 128, 1, 2, 5.93f, {0.309f, 0.793f}, 15.1f, run_gemm_ring<1, 2, 2, 3, false>},
+    {F_RING, 64, 256, 1, 1, 5.70f, {0.755f}, 13.0f, run_gemm_ring<1, 4, 1, 3, false>},
+    {F_RING, 128, 128, 1, 1, 4.40f, {0.534f}, 11.8f, run_gemm_ring<2, 2, 2, 3, false>},
+    {F_RING, 128, 256, 1, 1, 4.39f, {1.013f}, 10.7f, run_gemm_ring<2, 4, 1, 3, false>},
+    {F_RING, 256, 128, 1, 1, 3.87f, {0.935f}, 10.9f, run_gemm_ring<4, 2, 1, 3, false>},
+    {F_W4, 256, 256, 1, 1, 1.40f, {1.770f}, 7.9f, run_w4},
+};
+// several groups
+static const GemmForm kFormsG[] = {
+    {F_SK, 16, 32, 4, 2, 3.50f, {0.535f, 1.343f}, 20.0f, run_gemm_sk<2, 1, 4, 3>},
+    {F_SK, 32, 32, 8, 1, 3.23f, {1.383f}, 11.4f, run_gemm_sk<2, 2, 8, 2>},
+    {F_SK, 32, 64, 4, 1, 3.55f, {1.343f}, 20.0f, run_gemm_sk<4, 2, 4, 2>},
+    {F_RING, 64, 64, 1, 2, 4.71f, {0.701f, 0.758f}, 14.0f, run_gemm_ring<1, 1, 1, 4, true>},
+    {F_RING, 64, 128, 1, 2, 5.04f, {0.593f, 1.028f}, 12.7f, run_gemm_ring<1, 2, 1, 3, true>},
+    {F_RING, 64, 256, 1, 1, 4.91f, {0.795f}, 11.6f, run_gemm_ring<1, 4, 1, 3, true>},
+    {F_RING, 128, 128, 1, 1, 4.93f, {0.677f}, 10.0f, run_gemm_ring<2, 2, 1, 4, true>},
+    {F_RING, 128, 256, 1, 1, 4.05f, {1.095f}, 9.0f, run_gemm_ring<2, 4, 1, 3, true>},
+    {F_RING, 256, 128, 1, 1, 4.77f, {0.964f}, 9.2f, run_gemm_ring<4, 2, 1, 3, true>},
+    {F_RS, 256, 128, 1, 1, 6.23f, {0.961f}, 8.0f, run_rs},
+};
+// whether the form takes the shape (K and the groups in 128-byte stages are the caller's check)
+static bool form_takes(const GemmForm& f, const GemmArgs& a) {
+    if (a.N % f.bn) return false;
+    switch (f.kind) {
+        case F_W4: return a.M >= 512 && a.K >= 2 * kW4K;
+        case F_RS: return a.M >= 512 && a.K % 256 == 0;
+        // three stages of 384 rows leave room for the scales of 10 groups
+        case F_RING: return f.bm + f.bn < 384 || a.ng <= 10;
+        default: return true;
+    }
+}
+static float form_cost(const GemmForm& f, const GemmArgs& a, int cus) {
+    const long nb = (long)(a.N / f.bn) * ((a.M + f.bm - 1) / f.bm), n = (nb + cus - 1) / cus;
+    const float per = (float)(n / f.occ) * f.t[f.occ - 1] + (n % f.occ ? f.t[n % f.occ - 1] : 0.0f);
+    const float stages = (float)(a.K / 128) / f.ks, kb = (float)a.K * 1e-6f;
+    return f.a + fmaxf(stages * per, fmaxf((float)nb * (f.bm + f.bn) * kb / f.bw, (float)a.N * kb / 4.9f));
+}
 int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, float alpha, const int8_t* x,
                     const float* sx, int M, void* y, int ldy, int out_bf16, const void* res, int ldr, int res_bf16,
                     float rs, hipStream_t s, const AlphaSel* asel) {
@@ -652,53 +1103,33 @@ int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, floa
     a.M = M; a.N = N; a.K = K; a.gs = gs; a.ng = K / gs; a.ldy = ldy; a.ldr = ldr;
     a.out_bf16 = out_bf16; a.res_bf16 = res_bf16;
     if (asel) a.asel = *asel;
-    // Weight tiles of 128 rows (256-row tiles need 433 registers per lane, one block per CU, and
-    // measured 1-8% slower). Token tiles of 256 (8 waves, one block per CU, a 5-stage ring) from
-    // 512 tokens on: a third fewer bytes per MAC through the CU's load path; else 128 (4 waves,
-    // two blocks per CU, a 4-stage ring, or 3 when 17+ groups' scales take the room).
-    // One group over the whole K: 256 x 256 tiles when their launch takes fewer tile rounds on the
-    // CUs, counting a round of 256 x 256 tiles as 1.4 rounds of the rs kernel's 256 x 128 tiles
-    // (measured per round at 4096 x 16384 x 5120: 90 and 63 us); with too few tiles for the CUs
-    // the narrower tiles keep more of them busy. Q27X_GEMM_W4 = 1 / 0 takes / avoids them wherever
-    // the shape allows (tests of the kernel at small shapes, measurements).
-    if (M >= 512 && a.ng == 1 && N % kW4B == 0 && K % kW4K == 0 && K >= 2 * kW4K &&
-        (long)(M > N ? M : N) * K < (1L << 31) && (long)M * ldy < (1L << 30) && (!res || (long)M * ldr < (1L << 30))) {
-        const long mt = (M + 255) / 256, g = gemm_cus();
-        const long rw = ((long)(N / kW4B) * mt + g - 1) / g, ro = ((long)(N / kGN) * mt + g - 1) / g;
-        const char* f = getenv("Q27X_GEMM_W4");
-        const bool force = f && f[0] == '1' && !f[1], avoid = f && f[0] == '0' && !f[1];
-        if (force || (!avoid && rw * 14 < ro * 10)) {
-            const dim3 grid((unsigned)((N / kW4B) * mt));
-            const int rm = !res ? 0 : res_bf16 ? 2 : 1;
-            if (out_bf16) {
-                if (rm == 0) hipLaunchKernelGGL((k_gemm_i8g_w4<0, true>), grid, dim3(512), 0, s, a);
-                else if (rm == 1) hipLaunchKernelGGL((k_gemm_i8g_w4<1, true>), grid, dim3(512), 0, s, a);
-                else hipLaunchKernelGGL((k_gemm_i8g_w4<2, true>), grid, dim3(512), 0, s, a);
-            } else {
-                if (rm == 0) hipLaunchKernelGGL((k_gemm_i8g_w4<0, false>), grid, dim3(512), 0, s, a);
-                else if (rm == 1) hipLaunchKernelGGL((k_gemm_i8g_w4<1, false>), grid, dim3(512), 0, s, a);
-                else hipLaunchKernelGGL((k_gemm_i8g_w4<2, false>), grid, dim3(512), 0, s, a);
-            }
-            Q27X_HIP(hipGetLastError());
-            return Q27X_OK;
-        }
-    }
-    if (M >= 512 && K % 256 == 0 && gs % 128 == 0 && (long)M * ldy < (1L << 30) &&
+    // Whole 128-byte stages and 32-bit element offsets: the form that costs least. Q27X_GEMM_W4 = 1 / 0 takes /
+    // avoids the 256 x 256 tiles, Q27X_GEMM_FORM = i takes form i of the list, wherever the shape allows (tests of
+    // the kernels at small shapes, measurements).
+    if (K % 128 == 0 && gs % 128 == 0 && (long)(M > N ? M : N) * K < (1L << 31) && (long)M * ldy < (1L << 30) &&
         (!res || (long)M * ldr < (1L << 30))) {
-        const unsigned mt = (unsigned)((M + 255) / 256);
-        const size_t scl = (size_t)(256 + kGN) * a.ng * sizeof(float);
-        const dim3 grid((unsigned)(N / kGN) * mt);
-        const int rm = !res ? 0 : res_bf16 ? 2 : 1;
-        if (out_bf16) {
-            if (rm == 0) hipLaunchKernelGGL((k_gemm_i8g_rs<0, true>), grid, dim3(512), scl, s, a);
-            else if (rm == 1) hipLaunchKernelGGL((k_gemm_i8g_rs<1, true>), grid, dim3(512), scl, s, a);
-            else hipLaunchKernelGGL((k_gemm_i8g_rs<2, true>), grid, dim3(512), scl, s, a);
-        } else {
-            if (rm == 0) hipLaunchKernelGGL((k_gemm_i8g_rs<0, false>), grid, dim3(512), scl, s, a);
-            else if (rm == 1) hipLaunchKernelGGL((k_gemm_i8g_rs<1, false>), grid, dim3(512), scl, s, a);
-            else hipLaunchKernelGGL((k_gemm_i8g_rs<2, false>), grid, dim3(512), scl, s, a);
+        const GemmForm* forms = a.ng == 1 ? kFormsK : kFormsG;
+        const int nf = a.ng == 1 ? (int)(sizeof kFormsK / sizeof kFormsK[0]) : (int)(sizeof kFormsG / sizeof kFormsG[0]);
+        const char* ew = getenv("Q27X_GEMM_W4");
+        const char* ef = getenv("Q27X_GEMM_FORM");
+        const bool force = ew && ew[0] == '1' && !ew[1], avoid = ew && ew[0] == '0' && !ew[1];
+        const int want = ef && *ef ? atoi(ef) : -1;
+        const GemmForm* best = nullptr;
+        float cost = 0.0f;
+        for (int i = 0; i < nf; ++i) {
+            const GemmForm& f = forms[i];
+            if (!form_takes(f, a) || (avoid && f.kind == F_W4)) continue;
+            const float c = (i == want || (force && f.kind == F_W4)) ? -1.0f : form_cost(f, a, gemm_cus());
+            if (!best || c < cost) { best = &f; cost = c; }
         }
-    } else if (M >= 512) {
+        if (best) return best->run(a, s);
+    } else if (M >= 512 && K % 256 == 0 && gs % 128 == 0 && (long)M * ldy < (1L << 30) && (!res || (long)M * ldr < (1L << 30))) {
+        return run_rs(a, s);                                         // 2 GiB of codes and more: 64-bit addresses
+    }
+    // other shapes (K or the groups not in 128-byte stages): 64-byte stages, token tiles of 256 (8 waves, one block
+    // per CU, a 5-stage ring) from 512 tokens on, else 128 (4 waves, two blocks per CU, a 4-stage ring, or 3 when 17+
+    // groups' scales take the room)
+    if (M >= 512) {
         const unsigned mt = (unsigned)((M + 255) / 256);
         const size_t scl = (size_t)(256 + kGN) * a.ng * sizeof(float);
         hipLaunchKernelGGL((k_gemm_i8g<256, 5>), dim3((unsigned)(N / kGN) * mt), dim3(512), scl, (hipStream_t)s, a);

@@ -110,6 +110,13 @@ __device__ __forceinline__ void lds_dma16(const void* g, uint32_t lds) {
                  : "=&s"(save) : "s"(lds), "v"(g) : "memory");
 }
 
+// lds_dma16 from a wave-uniform base and a 32-bit offset per lane
+__device__ __forceinline__ void lds_dma16_at(const void* base, uint32_t off, uint32_t lds) {
+    uint32_t save;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(save) : "s"(lds), "v"(off), "s"(base) : "memory");
+}
 // The same for 4 bytes per lane: lane l's word from g lands at LDS byte address lds + 4 l.
 __device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds) {
     uint32_t save;

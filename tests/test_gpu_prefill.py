@@ -70,6 +70,14 @@ def test_tiny_prefill_gemm_matches_oracle(gpu, O, n, chunk, gs):
     run_case(gpu, O, gpu.tiny_config(spec_k=2, pf_gs=gs), n, 3, chunk)
 
 
+@pytest.mark.parametrize("form,gs", [(1, 0), (6, 0), (8, 0), (10, 0), (2, 1024), (8, 1024)])
+def test_tiny_prefill_gemm_forms_match_oracle(gpu, O, monkeypatch, form, gs):
+    """Split-K, ring and 256-token GEMM forms (Q27X_GEMM_FORM) in the prefill's epilogue forms: fp32 and bf16
+    outputs, fp32 and bf16 residuals, the stacked matrices' scales."""
+    monkeypatch.setenv("Q27X_GEMM_FORM", str(form))
+    run_case(gpu, O, gpu.tiny_config(spec_k=2, pf_gs=gs), 150, 2, None)
+
+
 def test_tiny_wide_group_swiglu_prefill_matches_oracle(gpu, O):
     """inter 5120 with whole-K groups: the down projection's input is quantized per (token, 5120)
     by the wide-group SwiGLU kernel (values held in registers: 1280 quads on 1024 threads, the

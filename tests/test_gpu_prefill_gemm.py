@@ -94,6 +94,40 @@ def test_gemm_i8g_wide_tiles(gpu, O, monkeypatch, M, N, K, with_res):
     same(f"wide-tile gemm {M}x{N}x{K}", y, oracle_gemm(O, w, sw, x, sx, K, 0.8125, res, 1.0))
 
 
+# the launch forms in the order of the launcher's lists: (tokens, weight rows) of a tile; (256, 256) and the last
+# grouped form take 512 tokens and more
+FORMS_K = [(16, 32), (32, 32), (32, 32), (32, 64), (64, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256),
+           (256, 128), (256, 256)]
+FORMS_G = [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 128)]
+
+
+@pytest.mark.parametrize("grouped,form", [(0, i) for i in range(12)] + [(1, i) for i in range(10)])
+def test_gemm_i8g_forms(gpu, O, monkeypatch, grouped, form):
+    """Every launch form (Q27X_GEMM_FORM) at the edges of its tiles and K stages: one token, one past a tile,
+    several ragged tiles; one K stage, odd counts, more groups than fit a phase (17 of 1024, 20 of 128)."""
+    monkeypatch.setenv("Q27X_GEMM_FORM", str(form))
+    bm, bn = (FORMS_G if grouped else FORMS_K)[form]
+    if grouped:
+        shapes = [(1, 256, 256, 128), (bm + 1, 512, 2560, 128), (2 * bm + 5, 256, 1152, 384), (37, 256, 17408, 1024)]
+        if form == 9:
+            shapes = [(513, 128, 512, 128), (600, 256, 2560, 128)]
+    else:
+        shapes = [(1, 256, 128, 128), (bm, 512, 384, 384), (bm + 1, 256, 1152, 1152), (2 * bm + 5, 512, 640, 640),
+                  (3, 256, 17408, 17408)]
+        if form == 11:
+            shapes = [(512, 256, 256, 256), (769, 512, 1152, 1152)]
+    for M, N, K, gs in shapes:
+        rng = np.random.default_rng(0x51E70600 + 100 * form + grouped + M + K)
+        ng = K // gs
+        w, x = codes(rng, (N, K)), codes(rng, (M, K))
+        w[0], x[0] = 127, -127
+        sw = rng.uniform(1e-4, 2e-3, (N, ng)).astype(np.float32)
+        sx = rng.uniform(1e-3, 5e-2, (M, ng)).astype(np.float32)
+        res = rng.standard_normal((M, N)).astype(np.float32) if M & 1 else None
+        y = gpu_gemm(gpu, w, sw, x, sx, gs, 0.8125, res, 1.0)
+        same(f"form {form}: {M}x{N}x{K}/{gs}", y, oracle_gemm(O, w, sw, x, sx, gs, 0.8125, res, 1.0))
+
+
 @pytest.mark.parametrize("gs", [5120, 1024])
 def test_gemm_i8g_full_shape_sampled(gpu, O, gs):
     # the prefill shape of gate (M = 4096 tokens, N = 17408, K = 5120) with whole-K groups (the
