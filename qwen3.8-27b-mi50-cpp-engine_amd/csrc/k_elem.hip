@@ -53,22 +53,43 @@ int launch_norm(const NormArgs& a, int nr, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- R5 activation quantizer
+// Four values per thread (one 8-byte load, one 4-byte store), a quantization group on a quad of lanes: a row of a few
+// thousand values is a handful of blocks, so the launch is one memory round trip plus its arithmetic, and a thread
+// per group (16 two-byte loads, 16 byte stores) was slower: 3 x 17408: 4.6 -> 3.8 us. VEC = 0 is that form, for
+// rows that are not 8-byte (codes: 4-byte) aligned.
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_quant_rows(const uint16_t* __restrict__ x, int xstride, int8_t* __restrict__ xq,
                                                     int qstride, float* __restrict__ xs, int sstride, int n, float g) {
     const int r = blockIdx.y;
-    const int gi = blockIdx.x * 256 + threadIdx.x;
-    const int k0 = gi * 16;
-    if (k0 >= n) return;
-    const uint16_t* xr = x + (size_t)r * xstride + k0;
-    float v[16], mx = 0.0f;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if constexpr (VEC) {
+        const int k0 = 4 * i, kc = k0 < n ? k0 : 0;     // (every lane of a quad takes part in its max)
+        const uint2 w = *(const uint2*)(x + (size_t)r * xstride + kc);
+        const float v[4] = {__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xFFFF0000u), __uint_as_float(w.y << 16),
+                            __uint_as_float(w.y & 0xFFFF0000u)};
+        float mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { v[j] = bf2f(xr[j]); mx = fmaxf(mx, fabsf(v[j])); }
-    const float s = mx * g * (1.0f / 127.0f);
-    const float inv = (s > 0.0f) ? (g / s) : 0.0f;
-    xs[(size_t)r * sstride + gi] = s;
-    int8_t* q = xq + (size_t)r * qstride + k0;
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, fabsf(v[j]));
+        mx = max_quad(mx);
+        const float s = mx * g * (1.0f / 127.0f);
+        const float inv = (s > 0.0f) ? (g / s) : 0.0f;
+        if (k0 >= n) return;
+        if ((i & 3) == 0) xs[(size_t)r * sstride + (i >> 2)] = s;
+        *(uint32_t*)(xq + (size_t)r * qstride + k0) = pack4(qcode(v[0], inv), qcode(v[1], inv), qcode(v[2], inv), qcode(v[3], inv));
+    } else {
+        const int k0 = i * 16;
+        if (k0 >= n) return;
+        const uint16_t* xr = x + (size_t)r * xstride + k0;
+        float v[16], mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) q[j] = qcode(v[j], inv);
+        for (int j = 0; j < 16; ++j) { v[j] = bf2f(xr[j]); mx = fmaxf(mx, fabsf(v[j])); }
+        const float s = mx * g * (1.0f / 127.0f);
+        const float inv = (s > 0.0f) ? (g / s) : 0.0f;
+        xs[(size_t)r * sstride + i] = s;
+        int8_t* q = xq + (size_t)r * qstride + k0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) q[j] = qcode(v[j], inv);
+    }
 }
 int launch_quant_rows(const uint16_t* x, int xstride, int8_t* xq, int qstride, float* xs, int sstride, int n,
                       float in_scale, int nrows, hipStream_t s) {
@@ -76,33 +97,54 @@ int launch_quant_rows(const uint16_t* x, int xstride, int8_t* xq, int qstride, f
         set_error("quant_rows: bad arguments (n=%d nrows=%d)", n, nrows);
         return Q27X_E_ARG;
     }
-    const int groups = n >> 4;
-    hipLaunchKernelGGL(k_quant_rows, dim3((groups + 255) / 256, nrows), dim3(256), 0, s, x, xstride, xq, qstride, xs,
-                       sstride, n, 1.0f / in_scale);
+    const bool vec = !((uintptr_t)x & 7) && !((uintptr_t)xq & 3) && (nrows == 1 || !((xstride & 3) | (qstride & 3)));
+    const int per = vec ? 4 : 16;
+    const dim3 grid((n / per + 255) / 256, nrows);
+    if (vec) hipLaunchKernelGGL(k_quant_rows<true>, grid, dim3(256), 0, s, x, xstride, xq, qstride, xs, sstride, n, 1.0f / in_scale);
+    else hipLaunchKernelGGL(k_quant_rows<false>, grid, dim3(256), 0, s, x, xstride, xq, qstride, xs, sstride, n, 1.0f / in_scale);
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }
 
 // ---------------------------------------------------------------- R16 SwiGLU + quantize
+// As k_quant_rows: four outputs per thread, a group on a quad (8 x 17408: 6.8 -> 4.9 us; the exponentials of 16
+// outputs one after another were most of a thread's time). VEC = 0: rows that are not 16-byte aligned.
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_swiglu(const float* __restrict__ G, const float* __restrict__ U, int stride,
                                                 int8_t* __restrict__ xq, float* __restrict__ xs, int n, float gs) {
+    constexpr int PT = VEC ? 4 : 16;
     const int r = blockIdx.y;
-    const int gi = blockIdx.x * 256 + threadIdx.x;
-    if (gi * 16 >= n) return;
-    const size_t base = (size_t)r * stride + (size_t)gi * 16;
-    float v[16], mx = 0.0f;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (!VEC && i * PT >= n) return;
+    const int k0 = i * PT < n ? i * PT : 0;
+    const size_t base = (size_t)r * stride + (size_t)k0;
+    float a[PT], u[PT], v[PT], mx = 0.0f;
+    if constexpr (VEC) {
+        const float4 a4 = *(const float4*)(G + base), u4 = *(const float4*)(U + base);
+        a[0] = a4.x; a[1] = a4.y; a[2] = a4.z; a[3] = a4.w;
+        u[0] = u4.x; u[1] = u4.y; u[2] = u4.z; u[3] = u4.w;
+    } else {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const float a = G[base + j];
-        const float sw = a / (1.0f + qexp(-a));
-        v[j] = sw * U[base + j] * gs;
+        for (int j = 0; j < PT; ++j) { a[j] = G[base + j]; u[j] = U[base + j]; }
+    }
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+        const float sw = a[j] / (1.0f + qexp(-a[j]));
+        v[j] = sw * u[j] * gs;
         mx = fmaxf(mx, fabsf(v[j]));
     }
+    if (VEC) mx = max_quad(mx);
     const float sc = mx * (1.0f / 127.0f);
     const float inv = (sc > 0.0f) ? (1.0f / sc) : 0.0f;
-    xs[(size_t)r * (n >> 4) + gi] = sc;
+    if (VEC && i * PT >= n) return;
+    if (!VEC || (i & 3) == 0) xs[(size_t)r * (n >> 4) + (k0 >> 4)] = sc;
+    int8_t* q = xq + (size_t)r * n + k0;
+    if constexpr (VEC) {
+        *(uint32_t*)q = pack4(qcode(v[0], inv), qcode(v[1], inv), qcode(v[2], inv), qcode(v[3], inv));
+    } else {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) xq[(size_t)r * n + (size_t)gi * 16 + j] = qcode(v[j], inv);
+        for (int j = 0; j < PT; ++j) q[j] = qcode(v[j], inv);
+    }
 }
 int launch_swiglu(const float* g, const float* u, int stride, int8_t* xq, float* xs, int n, float in_scale, int nr,
                   hipStream_t s) {
@@ -110,31 +152,67 @@ int launch_swiglu(const float* g, const float* u, int stride, int8_t* xq, float*
         set_error("swiglu: bad arguments");
         return Q27X_E_ARG;
     }
-    hipLaunchKernelGGL(k_swiglu, dim3((n / 16 + 255) / 256, nr), dim3(256), 0, s, g, u, stride, xq, xs, n,
-                       1.0f / in_scale);
+    const bool vec = !(((uintptr_t)g | (uintptr_t)u) & 15) && !((uintptr_t)xq & 3) && (nr == 1 || !(stride & 3));
+    const dim3 grid((n / (vec ? 4 : 16) + 255) / 256, nr);
+    if (vec) hipLaunchKernelGGL(k_swiglu<true>, grid, dim3(256), 0, s, g, u, stride, xq, xs, n, 1.0f / in_scale);
+    else hipLaunchKernelGGL(k_swiglu<false>, grid, dim3(256), 0, s, g, u, stride, xq, xs, n, 1.0f / in_scale);
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }
 
 // ---------------------------------------------------------------- R8 weight quantizer / generator
-// One thread per group of 64: sc = mx/127, q = rint(v/sc) (src/q27_nvfp4.hip:4259-4289).
+// Per group of 64: sc = mx/127, q = rint(v/sc) (src/q27_nvfp4.hip:4259-4289). Bound by memory: 16 lanes hold a group
+// (16-byte loads, 4-byte stores, both contiguous over the wave), kQwU groups' loads in flight per thread. A thread
+// per group read 256 bytes of its own, 64 lines per wave load: 16384 x 5120 took 313 us, now 75 (5.6 TB/s).
+// VEC = 0 is that form, for weights that are not 16-byte (codes: 4-byte) aligned.
+constexpr int kQwU = 4;
+template <bool VEC>
 __global__ __launch_bounds__(256) void k_quant_w(const float* __restrict__ w, int rows, int K, int8_t* __restrict__ wq,
                                                  float* __restrict__ ws) {
-    const long long gi = (long long)blockIdx.x * 256 + threadIdx.x;
     const int ng = K >> 6;
-    if (gi >= (long long)rows * ng) return;
-    const float* src = w + (size_t)gi * 64;
-    float mx = 0.0f;
-    for (int j = 0; j < 64; ++j) mx = fmaxf(mx, fabsf(src[j]));
-    const float sc = mx * (1.0f / 127.0f);
-    const float inv = (sc > 0.0f) ? (1.0f / sc) : 0.0f;
-    ws[gi] = sc;
-    for (int j = 0; j < 64; ++j) wq[(size_t)gi * 64 + j] = qcode(src[j], inv);
+    const long long n = (long long)rows * ng;           // groups
+    if constexpr (VEC) {
+        const int l = threadIdx.x & 15;
+        const long long g0 = (long long)blockIdx.x * (16 * kQwU) + (threadIdx.x >> 4);
+        float4 v[kQwU];
+#pragma unroll
+        for (int u = 0; u < kQwU; ++u) {
+            const long long g = g0 + 16 * u < n ? g0 + 16 * u : n - 1;
+            v[u] = *(const float4*)(w + (size_t)g * 64 + 4 * l);
+        }
+#pragma unroll
+        for (int u = 0; u < kQwU; ++u) {
+            const long long g = g0 + 16 * u;
+            float mx = fmaxf(fmaxf(0.0f, fabsf(v[u].x)), fabsf(v[u].y));
+            mx = fmaxf(fmaxf(mx, fabsf(v[u].z)), fabsf(v[u].w));
+            mx = max_xor(mx, 16);
+            const float sc = mx * (1.0f / 127.0f);
+            const float inv = (sc > 0.0f) ? (1.0f / sc) : 0.0f;
+            if (g < n) {
+                if (l == 0) ws[g] = sc;
+                *(uint32_t*)(wq + (size_t)g * 64 + 4 * l) =
+                    pack4(qcode(v[u].x, inv), qcode(v[u].y, inv), qcode(v[u].z, inv), qcode(v[u].w, inv));
+            }
+        }
+    } else {
+        const long long gi = (long long)blockIdx.x * 256 + threadIdx.x;
+        if (gi >= n) return;
+        const float* src = w + (size_t)gi * 64;
+        float mx = 0.0f;
+        for (int j = 0; j < 64; ++j) mx = fmaxf(mx, fabsf(src[j]));
+        const float sc = mx * (1.0f / 127.0f);
+        const float inv = (sc > 0.0f) ? (1.0f / sc) : 0.0f;
+        ws[gi] = sc;
+        for (int j = 0; j < 64; ++j) wq[(size_t)gi * 64 + j] = qcode(src[j], inv);
+    }
 }
 int launch_quant_w(const float* w, int rows, int K, int8_t* wq, float* ws, hipStream_t s) {
     if (!w || !wq || !ws || rows < 1 || K < 64 || (K & 63)) { set_error("quant_w: bad arguments"); return Q27X_E_ARG; }
     const long long ng = (long long)rows * (K >> 6);
-    hipLaunchKernelGGL(k_quant_w, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s, w, rows, K, wq, ws);
+    if (!((uintptr_t)w & 15) && !((uintptr_t)wq & 3))
+        hipLaunchKernelGGL(k_quant_w<true>, dim3((unsigned)((ng + 16 * kQwU - 1) / (16 * kQwU))), dim3(256), 0, s, w, rows, K, wq, ws);
+    else
+        hipLaunchKernelGGL(k_quant_w<false>, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s, w, rows, K, wq, ws);
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }

@@ -10,32 +10,40 @@ namespace q27x {
 // bf16 rows [M][ld] -> per-(token, group) codes [M][K] and scales [M][K / gs] (the quantizer of
 // k_quant_tok_grp on the rows' float values with gq = 1/in_scale: sc = max|v| gq / 127,
 // qi = sc > 0 ? gq / sc : 0).
-// One 256-thread block per (group, token), four values per thread per 1024 columns.
-__global__ __launch_bounds__(256) void k_pf_quant_bf16(const uint16_t* __restrict__ x, int ld, int K, int gs,
-                                                       int8_t* __restrict__ xq, float* __restrict__ xs, float gq) {
+// One block per (group, token), the group's values in registers (quant_group); NV = 0: groups wider than 20480, in
+// two passes over the row.
+template <int T, int NV>
+__global__ __launch_bounds__(T) void k_pf_quant_bf16(const uint16_t* __restrict__ x, int ld, int K, int gs,
+                                                     int8_t* __restrict__ xq, float* __restrict__ xs, float gq) {
     const int g = blockIdx.x, tok = blockIdx.y, t = threadIdx.x, ng = K / gs;
-    __shared__ float red[4];
+    __shared__ float red[T / 64];
     const uint16_t* row = x + (size_t)tok * ld + (size_t)g * gs;
-    float mx = 0.0f;
-    for (int k = 4 * t; k < gs; k += 1024) {
-        const uint2 u = *(const uint2*)(row + k);
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(__uint_as_float(u.x << 16)), fabsf(__uint_as_float(u.x & 0xFFFF0000u))),
-                             fmaxf(fabsf(__uint_as_float(u.y << 16)), fabsf(__uint_as_float(u.y & 0xFFFF0000u)))));
-    }
-    mx = max_xor(mx, 64);
-    if ((t & 63) == 0) red[t >> 6] = mx;
-    __syncthreads();
-    const float m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float sc = m * gq * (1.0f / 127.0f), qi = (sc > 0.0f) ? gq / sc : 0.0f;
-    if (t == 0) xs[(size_t)tok * ng + g] = sc;
     int8_t* out = xq + (size_t)tok * K + (size_t)g * gs;
-    for (int k = 4 * t; k < gs; k += 1024) {
+    auto quad = [&](int k) __attribute__((always_inline)) {
         const uint2 u = *(const uint2*)(row + k);
-        const uint32_t pk = (uint32_t)(uint8_t)qcode(__uint_as_float(u.x << 16), qi) |
-                            ((uint32_t)(uint8_t)qcode(__uint_as_float(u.x & 0xFFFF0000u), qi) << 8) |
-                            ((uint32_t)(uint8_t)qcode(__uint_as_float(u.y << 16), qi) << 16) |
-                            ((uint32_t)(uint8_t)qcode(__uint_as_float(u.y & 0xFFFF0000u), qi) << 24);
-        *(uint32_t*)(out + k) = pk;
+        return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xFFFF0000u), __uint_as_float(u.y << 16),
+                           __uint_as_float(u.y & 0xFFFF0000u));
+    };
+    if constexpr (NV > 0) {
+        quant_group<T, NV>(quad, gs, gq, out, xs + (size_t)tok * ng + g, red);
+    } else {
+        float mx = 0.0f;
+        for (int k = 4 * t; k < gs; k += 4 * T) {
+            const float4 v = quad(k);
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        }
+        mx = max_xor(mx, 64);
+        if ((t & 63) == 0) red[t >> 6] = mx;
+        __syncthreads();
+        float m = red[0];
+#pragma unroll
+        for (int w = 1; w < T / 64; ++w) m = fmaxf(m, red[w]);
+        const float sc = m * gq * (1.0f / 127.0f), qi = (sc > 0.0f) ? gq / sc : 0.0f;
+        if (t == 0) xs[(size_t)tok * ng + g] = sc;
+        for (int k = 4 * t; k < gs; k += 4 * T) {
+            const float4 v = quad(k);
+            *(uint32_t*)(out + k) = pack4(qcode(v.x, qi), qcode(v.y, qi), qcode(v.z, qi), qcode(v.w, qi));
+        }
     }
 }
 int launch_pf_quant_bf16(const uint16_t* x, int ld, int M, int K, int gs, float in_scale, int8_t* xq, float* xs,
@@ -45,8 +53,14 @@ int launch_pf_quant_bf16(const uint16_t* x, int ld, int M, int K, int gs, float 
         set_error("prefill quant: bad arguments (M %d, K %d, gs %d, ld %d)", M, K, gs, ld);
         return Q27X_E_ARG;
     }
-    hipLaunchKernelGGL(k_pf_quant_bf16, dim3((unsigned)(K / gs), (unsigned)M), dim3(256), 0, s, x, ld, K, gs, xq, xs,
-                       1.0f / in_scale);
+    const dim3 grid((unsigned)(K / gs), (unsigned)M);
+#define Q27X_QB(T, NV) hipLaunchKernelGGL((k_pf_quant_bf16<T, NV>), grid, dim3(T), 0, s, x, ld, K, gs, xq, xs, 1.0f / in_scale)
+    if (gs <= 1024) Q27X_QB(256, 1);
+    else if (gs <= 4096) Q27X_QB(256, 4);
+    else if (gs <= 6144) Q27X_QB(512, 3);
+    else if (gs <= 20480) Q27X_QB(1024, 5);
+    else Q27X_QB(256, 0);
+#undef Q27X_QB
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }

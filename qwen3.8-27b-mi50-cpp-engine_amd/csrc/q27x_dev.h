@@ -246,6 +246,40 @@ __device__ __forceinline__ int8_t qcode(float v, float inv) {
     c = c < -127 ? -127 : (c > 127 ? 127 : c);
     return (int8_t)c;
 }
+// four int8 codes in one word, the first in the low byte
+__device__ __forceinline__ uint32_t pack4(int8_t a, int8_t b, int8_t c, int8_t d) {
+    return (uint32_t)(uint8_t)a | ((uint32_t)(uint8_t)b << 8) | ((uint32_t)(uint8_t)c << 16) | ((uint32_t)(uint8_t)d << 24);
+}
+// One row's group of gs columns -> codes and scale (s = max gq / 127, inv = s > 0 ? gq / s : 0), its values held in
+// registers by the block: NV quads of T threads (gs <= 4 T NV), so the row is read once. ld(k): the four values from
+// column k (a multiple of 4) of the group; red: T / 64 floats of LDS.
+template <int T, int NV, typename LD>
+__device__ __forceinline__ void quant_group(LD ld, int gs, float gq, int8_t* out, float* sc_out, float* red) {
+    const int t = threadIdx.x;
+    float4 v[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int k = 4 * (t + T * u);
+        v[u] = k < gs ? ld(k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+    mx = max_xor(mx, 64);
+    if ((t & 63) == 0) red[t >> 6] = mx;
+    __syncthreads();
+    float m = red[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) m = fmaxf(m, red[w]);
+    const float sc = m * gq * (1.0f / 127.0f), qi = (sc > 0.0f) ? gq / sc : 0.0f;
+    if (t == 0) *sc_out = sc;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int k = 4 * (t + T * u);
+        if (k < gs) *(uint32_t*)(out + k) = pack4(qcode(v[u].x, qi), qcode(v[u].y, qi), qcode(v[u].z, qi), qcode(v[u].w, qi));
+    }
+}
 __device__ __forceinline__ uint4 ld_nt16(const void* p) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     const u32x4 v = __builtin_nontemporal_load((const u32x4*)p);

@@ -208,6 +208,54 @@ def test_swiglu_quant(gpu, O):
     same("swiglu scales", ds.download(np.float32, (nr, n // 16)), xs_o)
 
 
+@pytest.mark.parametrize("n,nr,off", [(16, 1, 0), (1040, 3, 0), (17408, 8, 0), (1040, 3, 1), (2064, 2, 2)])
+def test_quantizers_widths_and_alignment(gpu, O, n, nr, off):
+    """The activation and SwiGLU quantizers at one group, ragged block ends and full rows, and (off: elements the
+    rows start past an aligned address) in the form for rows that wide loads cannot take."""
+    X = gpu
+    rng = np.random.default_rng(n + off)
+    x = bf16_normal(rng, (nr, n), O=O)
+    x[0, :16] = 0
+    xq_o, xs_o = np.empty((nr, n), np.int8), np.empty((nr, n // 16), np.float32)
+    O.lib().q27o_quant_rows(x.ctypes.data, n, xq_o.ctypes.data, n, xs_o.ctypes.data, n // 16, n, 1.0, nr)
+    dx, dq, ds = dev(X, np.concatenate([np.zeros(off, np.uint16), x.ravel()])), X.DevBuf(nr * n + off), X.DevBuf(nr * n // 4)
+    X.call("q27x_quant_rows", dx.ptr + 2 * off, n, dq.ptr + off, n, ds.ptr, n // 16, n, 1.0, nr, None)
+    X.call("q27x_device_sync")
+    same("codes", dq.download(np.int8, (nr * n + off,))[off:].reshape(nr, n), xq_o)
+    same("scales", ds.download(np.float32, (nr, n // 16)), xs_o)
+    g, u = ((rng.standard_normal((nr, n)) * 2).astype(np.float32) for _ in range(2))
+    O.lib().q27o_swiglu_quant_rows(g.ctypes.data, u.ctypes.data, n, xq_o.ctypes.data, xs_o.ctypes.data, n, 1.0, nr)
+    dg, du = (dev(X, np.concatenate([np.zeros(off, np.float32), a.ravel()])) for a in (g, u))
+    X.call("q27x_swiglu_quant_rows", dg.ptr + 4 * off, du.ptr + 4 * off, n, dq.ptr + off, ds.ptr, n, 1.0, nr, None)
+    X.call("q27x_device_sync")
+    same("swiglu codes", dq.download(np.int8, (nr * n + off,))[off:].reshape(nr, n), xq_o)
+    same("swiglu scales", ds.download(np.float32, (nr, n // 16)), xs_o)
+
+
+@pytest.mark.parametrize("rows,K,off", [(1, 64, 0), (7, 576, 0), (33, 5120, 0), (7, 576, 1), (5, 1024, 2)])
+def test_quant_weights_widths_and_alignment(gpu, O, rows, K, off):
+    X = gpu
+    rng = np.random.default_rng(rows + K + off)
+    w = rng.standard_normal((rows, K)).astype(np.float32)
+    w[0, :64] = 0
+    wq_o, ws_o = np.empty((rows, K), np.int8), np.empty((rows, K // 64), np.float32)
+    O.lib().q27o_quant_weights_i8g64(w.ctypes.data, rows, K, wq_o.ctypes.data, ws_o.ctypes.data)
+    dw, dq, ds = dev(X, np.concatenate([np.zeros(off, np.float32), w.ravel()])), X.DevBuf(rows * K + off), X.DevBuf(rows * K // 16)
+    X.call("q27x_quant_weights_i8g64", dw.ptr + 4 * off, rows, K, dq.ptr + off, ds.ptr, None)
+    X.call("q27x_device_sync")
+    same("codes", dq.download(np.int8, (rows * K + off,))[off:].reshape(rows, K), wq_o)
+    same("scales", ds.download(np.float32, (rows, K // 64)), ws_o)
+    # ... and the GEMM's representation of them, in groups of 64 columns and of the whole K
+    for gs in (64, K):
+        wg_o, sg_o = np.empty((rows, K), np.int8), np.empty((rows, K // gs), np.float32)
+        O.lib().q27o_i8g64_to_grp(wq_o.ctypes.data, ws_o.ctypes.data, rows, K, gs, wg_o.ctypes.data, sg_o.ctypes.data)
+        dg, dsg = X.DevBuf(rows * K + off), X.DevBuf(rows * (K // gs) * 4)
+        X.call("q27x_i8g64_to_grp", dq.ptr + off, ds.ptr, rows, K, gs, dg.ptr + off, dsg.ptr, None)
+        X.call("q27x_device_sync")
+        same("group codes", dg.download(np.int8, (rows * K + off,))[off:].reshape(rows, K), wg_o)
+        same("group scales", dsg.download(np.float32, (rows, K // gs)), sg_o)
+
+
 @pytest.mark.parametrize("op,lo,hi", [(0, -110, 95), (1, -160, 130), (2, -0.99, 1e9), (3, -100, 100),
                                       (4, -100, 100), (5, -30, 30)])
 def test_math_bit_exact(gpu, O, op, lo, hi):

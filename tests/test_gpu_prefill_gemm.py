@@ -175,6 +175,21 @@ def test_quant_tok_groups(gpu, O, K, gs):
         b.free()
 
 
+@pytest.mark.parametrize("K,gs", [(64, 64), (2048, 2048), (4100, 4100), (6144, 6144), (6148, 6148), (20544, 20544)])
+def test_quant_tok_groups_widths(gpu, O, K, gs):
+    """A group per register form of the quantizer (up to 1024, 2048, 4096, 6144 and 20480 columns, and wider)."""
+    X = gpu
+    M = 3
+    x = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    xq_o, xs_o = np.empty((M, K), np.int8), np.empty((M, 1), np.float32)
+    O.lib().q27o_quant_tok_groups(x.ctypes.data, K, M, K, gs, xq_o.ctypes.data, xs_o.ctypes.data)
+    dx, dq, ds = X.DevBuf(array=x), X.DevBuf(M * K), X.DevBuf(M * 4)
+    X.call("q27x_quant_tok_groups", dx.ptr, K, M, K, gs, dq.ptr, ds.ptr, None)
+    X.call("q27x_device_sync")
+    same("codes", dq.download(np.int8, (M, K)), xq_o)
+    same("scales", ds.download(np.float32, (M, 1)), xs_o)
+
+
 @pytest.mark.parametrize("rows,K,gs,in_place", [(300, 5120, 1024, False), (64, 17408, 1024, True),
                                                 (128, 5120, 5120, False)])
 def test_i8g64_to_grp(gpu, O, rows, K, gs, in_place):
