@@ -9,6 +9,7 @@
 //   owns (split, kv head) for all rows and all GQA heads: K/V tile dequantised into LDS once,
 //   scores by 16-lane dot products, two-pass softmax in base 2, p.V in key order; the combine
 //   merges splits in order, applies sigmoid(gate) and quantises for o_proj.
+#include <algorithm>
 #include <mutex>
 
 #include "q27x_dev.h"
@@ -601,14 +602,17 @@ __global__ __launch_bounds__(HD) void k_attn_combine(AttnArgs a, int nr) {
 // 8 waves, on v_mfma_f32_16x16x4f32 (an instruction adds its four products one after another with
 // fused multiply-adds, so a chain of them is an fmaf loop). Bound by the fp32 matrix rate (157
 // TFLOP/s): the int8 K/V bytes are a third of that time at 48 query vectors.
-//   K/V: int8 tiles and their scales by LDS DMA, one split ahead in a second buffer, 16-byte chunk
-//     c of key row R in slot c ^ (R % (HD/16)), so the 16 keys of an operand read hit distinct
-//     banks; codes are widened and scaled as operands are read (an fp32 tile of 256-wide rows
-//     would not leave room, and costs a pass and a barrier of its own).
+//   K/V: int8 tiles and their scales by LDS DMA, 16-byte chunk c of key row R in slot
+//     c ^ (R % (HD/16)), so the 16 keys of an operand read hit distinct banks; codes are widened and
+//     scaled as operands are read (an fp32 tile of 256-wide rows would not leave room, and costs a
+//     pass and a barrier of its own). The next split's K is requested behind the scores, its V
+//     behind P.V.
 //   scores: wave (key tile kt, half h) runs chains 2h and 2h + 1 (its half of the dims) of all QT
-//     query tiles, the queries in registers for the whole launch; every wave has the same work at
-//     any QT. c0 + c1, c2 and c3 meet in LDS, where the softmax adds them.
+//     query tiles, the queries (bf16 pairs) in registers for the whole launch; every wave has the
+//     same work at any QT. The second half's waves add c2, then c3 to the first's c0 + c1 in LDS.
 //   P.V: wave w owns HD/128 16-dim tiles for all query tiles.
+// At most 128 registers and half of a CU's LDS, so two blocks share a CU and one's softmax and waits
+// are covered by the other's matrix work.
 constexpr int kGThreads = 512;
 // x, as a value the compiler cannot move out of the loop it is taken in
 __device__ __forceinline__ int opaque(int x) {
@@ -616,14 +620,14 @@ __device__ __forceinline__ int opaque(int x) {
     return x;
 }
 constexpr int kSpG = kSplit + 4;                 // score row stride (floats)
-// Dynamic LDS of a launch with QT query tiles: 2 x (K, V codes) | 2 x (K, V scales) | 3 score arrays
-// (the query stage before the first scores)
+// Dynamic LDS of a launch with QT query tiles: K, V codes | K, V scales | scores; the query stage before the
+// first split takes the room from the codes on
 template <int HD>
-__host__ __device__ constexpr size_t split_g_lds(int qt) {
-    return (size_t)4 * kSplit * HD + (size_t)4 * kSplit * (HD / 16) * 4 + (size_t)3 * qt * 16 * kSpG * 4;
+__host__ __device__ constexpr size_t split_g_lds(int qt, int nsc) {
+    return (size_t)2 * kSplit * HD + (size_t)2 * kSplit * nsc * 4 + (size_t)qt * 16 * kSpG * 4;
 }
 template <int HD, int QT>
-__global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) {
+__global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int nr) {
     warm_args(a);
     if (stopped(a.stop)) return;
     constexpr int NCH = HD / 16;                 // 16-byte chunks per key row; scales per row at most
@@ -641,12 +645,12 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
     const int ms = a.max_splits;
     const int gsh = __builtin_ctz(a.kv_group), nsc = HD >> gsh;     // kv_group is 16, 32 or 64
     extern __shared__ __attribute__((aligned(16))) int8_t gdyn[];
-    int8_t* kv8 = gdyn;                                             // [2][K | V][64][HD]
-    float* scl = (float*)(gdyn + 4 * kSplit * HD);                  // [2][K | V][64][nsc] (room for NCH)
-    float* sp = scl + 4 * kSplit * NCH;                             // [NQ][kSpG] c0 + c1, then p
-    float* sc2 = sp + NQ * kSpG;                                    // c2
-    float* sc3 = sc2 + NQ * kSpG;                                   // c3
-    __shared__ int sbad[2];                                         // per buffer: a hidden V row is not finite
+    const int8_t* k8 = gdyn;                                        // [64][HD]
+    const int8_t* v8 = gdyn + kSplit * HD;
+    const float* ksc = (const float*)(gdyn + 2 * kSplit * HD);      // [64][nsc]
+    const float* vsc = ksc + kSplit * nsc;
+    float* sp = (float*)(gdyn + 2 * kSplit * HD) + 2 * kSplit * nsc;   // [NQ][kSpG] scores, then p
+    __shared__ int sbad;                                            // a V row that some rows do not see is not finite
     const int t = threadIdx.x, lane = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int g4 = lane >> 4, j16 = lane & 15;
@@ -655,40 +659,44 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
     float* wl = wm + (size_t)nr * a.nq * ms;
     int s = blockIdx.x;
     if (s * kSplit >= Lmax) return;
-    // split s into buffer b: 1 KiB of codes per wave instruction (64 / NCH key rows), then one scale
-    // per lane; keys past the last read the split's first key (visible to every row that uses the
-    // split, so it adds nothing that is not there already)
-    const uint32_t kv_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)kv8;
-    const uint32_t scl_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)scl;
-    auto load_tile = [&](int sn, int b) __attribute__((always_inline)) {
+    // K (isv = 0) or V of split sn: 1 KiB of codes per wave instruction (64 / NCH key rows), then one scale per lane;
+    // keys past the last read the split's first key (visible to every row that uses the split, so it adds nothing
+    // that is not there already). Every wave issues the same number of transfers: kTI and the scales' nsc / 8 (1 or 2;
+    // with fewer than 8 instructions of scales some waves repeat others').
+    constexpr int kRPI = 64 / NCH, kNI = kSplit / kRPI, kTI = kNI / 8;
+    const uint32_t kv_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)gdyn;
+    const uint32_t scl_lds = kv_lds + 2 * kSplit * HD;
+    auto load_tile = [&](int sn, int isv) __attribute__((always_inline)) {
         const int k0 = sn * kSplit;
         const int nk = (Lmax - k0 < kSplit) ? (Lmax - k0) : kSplit;
-        constexpr int RPI = 64 / NCH, NI = kSplit / RPI;            // rows per instruction, instructions per matrix
         const int lane = opaque((int)threadIdx.x & 63);
 #pragma unroll
-        for (int i = 0; i < 2 * NI / 8; ++i) {
-            const int u = wv + 8 * i, isv = u / NI, R = (u % NI) * RPI + lane / NCH;
+        for (int i = 0; i < kTI; ++i) {
+            const int u = wv + 8 * i, R = u * kRPI + lane / NCH;
             const int c = (lane % NCH) ^ (R % NCH);
             const size_t off = (size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD + 16 * c;
             lds_dma16((isv ? a.vc : a.kc) + off,
-                      __builtin_amdgcn_readfirstlane(kv_lds + (uint32_t)((2 * b + isv) * kSplit * HD + 1024 * (u % NI))));
+                      __builtin_amdgcn_readfirstlane(kv_lds + (uint32_t)(isv * kSplit * HD + 1024 * u)));
         }
-        for (int u = wv; u < 2 * nsc; u += 8) {                     // nsc instructions of 64 scales per matrix
-            const int isv = u >= nsc, i = isv ? u - nsc : u;
-            const int f = 64 * i + lane, R = f >> (__builtin_ctz(HD) - gsh), c = f & (nsc - 1);
+        for (int i = wv; i < (nsc < 8 ? 8 : nsc); i += 8) {          // nsc instructions of 64 scales
+            const int j = i & (nsc - 1), f = 64 * j + lane, R = f >> (__builtin_ctz(HD) - gsh), c = f & (nsc - 1);
             const size_t off = (((size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD) >> gsh) + c;
             lds_dma4((isv ? a.vs : a.ks) + off,
-                     __builtin_amdgcn_readfirstlane(scl_lds + (uint32_t)((2 * b + isv) * kSplit * NCH + 64 * i) * 4u));
+                     __builtin_amdgcn_readfirstlane(scl_lds + (uint32_t)(isv * kSplit * nsc + 64 * j) * 4u));
         }
     };
-    load_tile(s, 0);
+    // all but the newest matrix's transfers of this wave have landed
+    auto wait_older = [&]() __attribute__((always_inline)) {
+        if (nsc > 8) __builtin_amdgcn_s_waitcnt(vmcnt_imm(kTI + 2));
+        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(kTI + 1));
+    };
     // queries: bf16 rows to LDS with dims 8 c + g and 8 c + 4 + g paired in word [row][g][c], then each
     // lane's values (query 16 qt + j16, dims HD/2 h + 4 s + g4) to registers
     const int kt = wv & 3, h = wv >> 2;
-    float q[QT][NS];
+    uint32_t q[QT][NS / 2];                          // values s (low half) and s + 1
     {
         constexpr int QS = HD / 2 + 4;                              // words per staged query row
-        uint32_t* sq = (uint32_t*)sp;
+        uint32_t* sq = (uint32_t*)gdyn;
         for (int i = t; i < NQ * (HD / 8); i += kGThreads) {
             const int qi = i / (HD / 8), c = i % (HD / 8);
             const int qc = qi < nqr ? qi : 0;                       // rows past nqr: computed, not stored
@@ -700,44 +708,35 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
             d[2 * (HD / 8)] = __builtin_amdgcn_perm(x.w, x.y, 0x05040100u);
             d[3 * (HD / 8)] = __builtin_amdgcn_perm(x.w, x.y, 0x07060302u);
         }
-        if (t == 0) sbad[0] = sbad[1] = 0;
+        if (t == 0) sbad = 0;
         __syncthreads();
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
             for (int m = 0; m < NS / 8; ++m) {
                 const uint4 x = *(const uint4*)(sq + (16 * qt + j16) * QS + g4 * (HD / 8) + (NS / 2) * h + 4 * m);
-                const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    q[qt][8 * m + 2 * e] = __uint_as_float(w[e] << 16);
-                    q[qt][8 * m + 2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
-                }
+                q[qt][4 * m] = x.x; q[qt][4 * m + 1] = x.y; q[qt][4 * m + 2] = x.z; q[qt][4 * m + 3] = x.w;
             }
+        __syncthreads();                                            // the query stage is read
     }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));                       // this wave's transfers have landed
-    __syncthreads();                                                // every wave's; the query stage is read
-    for (int b = 0; s * kSplit < Lmax; s += gridDim.x, b ^= 1) {
+    load_tile(s, 0);
+    load_tile(s, 1);
+    for (; s * kSplit < Lmax; s += gridDim.x) {
         const int k0 = s * kSplit;
         const int nk = (Lmax - k0 < kSplit) ? (Lmax - k0) : kSplit;
-        const int8_t* k8 = kv8 + (size_t)(2 * b) * kSplit * HD;
-        const int8_t* v8 = k8 + kSplit * HD;
-        const float* ksc = scl + (2 * b) * kSplit * NCH;
-        const float* vsc = ksc + kSplit * NCH;
-        // the block's next split: in flight through this split's work
-        if ((s + (int)gridDim.x) * kSplit < Lmax) load_tile(s + gridDim.x, b ^ 1);
-        // A value that is not finite in a V row that some of the block's rows do not see (p = 0)
-        // would reach them through the matrix cores: such splits take P.V key by key.
-        if (k0 + nk > pos0 + 1) {
-            const int kf = pos0 + 1 > k0 ? pos0 + 1 - k0 : 0;       // first key that row 0 does not see
-            for (int i = kf * nsc + t; i < nk * nsc; i += kGThreads)
-                if (!(fabsf(vsc[i]) < __builtin_huge_valf())) sbad[b] = 1;
-        }
+        const int sn = s + (int)gridDim.x;
+        const bool more = sn * kSplit < Lmax;                       // the block has another split
+        wait_older();                                               // this wave's K transfers have landed
+        __syncthreads();                                            // every wave's
         // (each phase takes the lane's indices anew: hoisted out of the loop, their addresses alone would
         // not fit the registers beside the queries)
         // ---- scores: lane 16 g + j supplies q(16 qt + j)[d] and k(16 kt + j)[d], d = HD/2 h + 4 s + g
         {
             const int ln = opaque(lane), g4 = ln >> 4, j16 = ln & 15;
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int i = 0; i < NS / 2; ++i) asm volatile("" : "+v"(q[qt][i]));   // (widened here, not ahead of the loop)
             const int key = 16 * kt + j16;
             v4f acc[QT][2];
 #pragma unroll
@@ -760,26 +759,43 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
 #pragma unroll
                     for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-                        for (int c = 0; c < 2; ++c)
-                            acc[qt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[qt][(NS / 2) * c + 4 * m + e], k[c][e],
-                                                                              acc[qt][c], 0, 0, 0);
+                        for (int c = 0; c < 2; ++c) {
+                            const uint32_t qw = q[qt][(NS / 4) * c + 2 * m + e / 2];
+                            acc[qt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                __uint_as_float(e & 1 ? qw & 0xFFFF0000u : qw << 16), k[c][e], acc[qt][c], 0, 0, 0);
+                        }
                 __builtin_amdgcn_sched_barrier(0);   // (all chunks widened ahead do not fit the registers)
             }
+            float* sr = sp + 4 * g4 * kSpG + key;
+            if (h == 0) {
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
+                for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int i = (16 * qt + 4 * g4 + r) * kSpG + key;
-                    if (h == 0) {
-                        sp[i] = acc[qt][0][r] + acc[qt][1][r];
-                    } else {
-                        sc2[i] = acc[qt][0][r];
-                        sc3[i] = acc[qt][1][r];
+                    for (int r = 0; r < 4; ++r) sr[(16 * qt + r) * kSpG] = acc[qt][0][r] + acc[qt][1][r];
+            }
+            __syncthreads();                                        // K is read, the first half's sums are there
+            if (more) load_tile(sn, 0);
+            if (h == 1) {
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int i = (16 * qt + r) * kSpG;
+                        sr[i] = (sr[i] + acc[qt][0][r]) + acc[qt][1][r];
                     }
-                }
+            }
         }
+        // V's transfers (older than the next K's) have landed for this wave, after the barrier for all
+        if (more) wait_older();
+        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __syncthreads();
-        if (t == 0) sbad[b ^ 1] = 0;                // (read in the split before, set at the earliest in the next)
+        // A value that is not finite in a V row that some of the block's rows do not see (p = 0)
+        // would reach them through the matrix cores: such splits take P.V key by key.
+        if (k0 + nk > pos0 + 1) {
+            const int kf = pos0 + 1 > k0 ? pos0 + 1 - k0 : 0;       // first key that row 0 does not see
+            for (int i = kf * nsc + t; i < nk * nsc; i += kGThreads)
+                if (!(fabsf(vsc[i]) < __builtin_huge_valf())) sbad = 1;
+        }
         // ---- split softmax as in k_attn_split: four queries of the wave at a time, lane 16 i + c holding
         // keys c, c + 16, c + 32, c + 48 of the pass's i-th; p of key k goes to position
         // 16 (k % 4) + k / 4 of the row, where a lane of P.V finds its 16 keys 4 s + g side by side
@@ -797,7 +813,7 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = qc * kSpG + j16 + 16 * e;
-                    x[e] = ((sp[i] + sc2[i]) + sc3[i]) * a.sl2e;
+                    x[e] = sp[i] * a.sl2e;
                     if (j16 + 16 * e < nv) m = fmaxf(m, x[e]);
                 }
                 m = max_xor(m, 16);
@@ -820,11 +836,8 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
             }
         }
         __syncthreads();
-        const int bad = sbad[b];
+        const int bad = sbad;
         // ---- o = sum_k p_k v_k: lane 16 g + j supplies p(16 qt + j)[4 s + g] and v(4 s + g)[16 dt + j]
-        // this wave's transfers of the next split have landed (waited for ahead of the stores below,
-        // which the count would include)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         float* ws = wo + ((size_t)(kvh * G) * ms + s) * HD;
         auto put = [&](int qi, int d, float o) __attribute__((always_inline)) {
             const int r = (int)((qi * gdiv) >> 16), g = qi - r * G;
@@ -884,7 +897,9 @@ __global__ __launch_bounds__(kGThreads) void k_attn_split_g(AttnArgs a, int nr) 
                 put(qi, d, ((o4[0] + o4[1]) + o4[2]) + o4[3]);
             }
         }
-        __syncthreads();                            // the split is consumed, the next one landed
+        __syncthreads();                            // the split is consumed
+        if (more) load_tile(sn, 1);
+        if (t == 0) sbad = 0;                       // (read before the barrier, set behind two more)
     }
 }
 
@@ -937,13 +952,14 @@ static int launch_split_g(const AttnArgs& a, int nr, hipStream_t s) {
         const void* f[4] = {(const void*)k_attn_split_g<HD, 1>, (const void*)k_attn_split_g<HD, 2>,
                             (const void*)k_attn_split_g<HD, 3>, (const void*)k_attn_split_g<HD, 4>};
         for (int i = 0; i < 4 && attr_e == hipSuccess; ++i)
-            attr_e = hipFuncSetAttribute(f[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_g_lds<HD>(i + 1));
+            attr_e = hipFuncSetAttribute(f[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_g_lds<HD>(i + 1, HD / 16));
     });
     Q27X_HIP(attr_e);
     const int qt = (nr * (a.nq / a.nkv) + 15) / 16;
-    const int bx = a.max_splits < kSplitBlocks / a.nkv ? a.max_splits : (kSplitBlocks / a.nkv > 0 ? kSplitBlocks / a.nkv : 1);
+    // two blocks share a CU; a block takes splits blockIdx.x + i gridDim.x
+    const int bx = std::min(a.max_splits, std::max(1, 2 * kSplitBlocks / a.nkv));
     const dim3 grid(bx, a.nkv, a.zrows ? (unsigned)((a.ztotal + a.zrows - 1) / a.zrows) : 1u);
-    const size_t lds = split_g_lds<HD>(qt);
+    const size_t lds = split_g_lds<HD>(qt, HD / a.kv_group);
     switch (qt) {
         case 1: hipLaunchKernelGGL((k_attn_split_g<HD, 1>), grid, dim3(kGThreads), lds, s, a, nr); break;
         case 2: hipLaunchKernelGGL((k_attn_split_g<HD, 2>), grid, dim3(kGThreads), lds, s, a, nr); break;
