@@ -1245,6 +1245,14 @@ int launch_gemv(const GemvArgs& a, int argmax_mode, int nr, int* nblocks_out, hi
 }
 
 // ---------------------------------------------------------------- argmax
+// The wave's best candidate in every lane: its largest value, the lowest index that holds it, and that candidate's
+// own value (of two zeros, its sign). Lanes without a candidate hold -inf and index ~0. All on lane swaps and DPP.
+__device__ __forceinline__ void wave_best(float& bv, uint32_t& bi) {
+    const float m = max_xor(bv, 64);
+    const uint32_t i = min_xor64(bv == m ? bi : 0xFFFFFFFFu);
+    bv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bv), __builtin_ctzll(__ballot(bi == i))));
+    bi = i;
+}
 __global__ __launch_bounds__(256) void k_argmax_final(const float* __restrict__ pval, const uint32_t* __restrict__ pidx,
                                                       int pstride, int nblocks, int32_t* __restrict__ idx,
                                                       float* __restrict__ val, const int* stop) {
@@ -1258,16 +1266,11 @@ __global__ __launch_bounds__(256) void k_argmax_final(const float* __restrict__ 
         const uint32_t ii = pidx[(size_t)n * pstride + i];
         if (ii != 0xFFFFFFFFu) am_merge(bv, bi, pval[(size_t)n * pstride + i], ii);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, o, 64);
-        if (oi != 0xFFFFFFFFu) am_merge(bv, bi, ov, oi);
-    }
+    wave_best(bv, bi);
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 0; w < 4; ++w) if (si[w] != 0xFFFFFFFFu) am_merge(bv, bi, sv[w], si[w]);
+        for (int w = 1; w < 4; ++w) if (si[w] != 0xFFFFFFFFu) am_merge(bv, bi, sv[w], si[w]);
         const bool none = (bi == 0xFFFFFFFFu);
         idx[n] = none ? 0 : (int32_t)bi;
         if (val) val[n] = none ? -__builtin_huge_valf() : bv;
@@ -1280,36 +1283,44 @@ int launch_argmax_final(const float* pval, const uint32_t* pidx, int pstride, in
     return Q27X_OK;
 }
 
+// Partials of kAmBlocks blocks per row of logits (non-finite filtered, ties -> lowest index), kAmU loads of a thread
+// requested together: a 62080-wide row is one memory round trip. (Loads one behind another and 12 crossbar shuffles
+// per block took 5.0 us; one block per row takes 8.7, its compares on a single CU.)
+constexpr int kAmBlocks = 64, kAmU = 4;
 __global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ logits, int n, int ld,
                                                      float* __restrict__ pval, uint32_t* __restrict__ pidx, int pstride) {
     const int r = blockIdx.y;
     const float* p = logits + (size_t)r * ld;
     float bv = -__builtin_huge_valf();
     uint32_t bi = 0xFFFFFFFFu;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const float v = p[i];
-        if (finitef(v)) am_merge(bv, bi, v, (uint32_t)i);
-    }
+    for (int i0 = blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += gridDim.x * 256 * kAmU) {
+        float v[kAmU];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, o, 64);
-        if (oi != 0xFFFFFFFFu) am_merge(bv, bi, ov, oi);
+        for (int u = 0; u < kAmU; ++u) {
+            const int i = i0 + u * (int)gridDim.x * 256;
+            v[u] = p[i < n ? i : i0];
+        }
+#pragma unroll
+        for (int u = 0; u < kAmU; ++u) {                // (ascending indices: a later equal value never wins)
+            const int i = i0 + u * (int)gridDim.x * 256;
+            if (i < n && finitef(v[u]) && v[u] > bv) { bv = v[u]; bi = (uint32_t)i; }
+        }
     }
     __shared__ float sv[4];
     __shared__ uint32_t si[4];
+    wave_best(bv, bi);
     if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 0; w < 4; ++w) if (si[w] != 0xFFFFFFFFu) am_merge(bv, bi, sv[w], si[w]);
+        for (int w = 1; w < 4; ++w) if (si[w] != 0xFFFFFFFFu) am_merge(bv, bi, sv[w], si[w]);
         pval[(size_t)r * pstride + blockIdx.x] = bv;
         pidx[(size_t)r * pstride + blockIdx.x] = bi;
     }
 }
 // module-static partials of the kernel-tier argmax (as the reference's g_q27_am_val/idx arena,
 // src/q27_elem.hip:221-222): 8 rows x 64 blocks
-__device__ float g_am_val[kMaxRows * 64];
-__device__ uint32_t g_am_idx[kMaxRows * 64];
+__device__ float g_am_val[kMaxRows * kAmBlocks];
+__device__ uint32_t g_am_idx[kMaxRows * kAmBlocks];
 int argmax_scratch(float** pv, uint32_t** pi) {
     Q27X_HIP(hipGetSymbolAddress((void**)pv, HIP_SYMBOL(g_am_val)));
     Q27X_HIP(hipGetSymbolAddress((void**)pi, HIP_SYMBOL(g_am_idx)));
@@ -1317,10 +1328,9 @@ int argmax_scratch(float** pv, uint32_t** pi) {
 }
 int launch_argmax_rows(const float* logits, int n, int ld, int nr, int32_t* idx, float* val, float* pval,
                        uint32_t* pidx, hipStream_t s) {
-    const int nb = 64;
-    hipLaunchKernelGGL(k_argmax_part, dim3(nb, nr), dim3(256), 0, s, logits, n, ld, pval, pidx, nb);
+    hipLaunchKernelGGL(k_argmax_part, dim3(kAmBlocks, nr), dim3(256), 0, s, logits, n, ld, pval, pidx, kAmBlocks);
     Q27X_HIP(hipGetLastError());
-    return launch_argmax_final(pval, pidx, nb, nb, nr, idx, val, nullptr, s);
+    return launch_argmax_final(pval, pidx, kAmBlocks, kAmBlocks, nr, idx, val, nullptr, s);
 }
 
 }  // namespace q27x

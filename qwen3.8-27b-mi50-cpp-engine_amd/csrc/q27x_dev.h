@@ -211,6 +211,18 @@ __device__ __forceinline__ float max_xor(float x, int width) {
     if (width >= 64) x = fmaxf(x, xor32(x));
     return x;
 }
+// min of an unsigned value over the wave, in every lane (the same lane pairs)
+__device__ __forceinline__ uint32_t min_xor64(uint32_t x) {
+    auto lo = [](uint32_t a, uint32_t b) { return a < b ? a : b; };
+    x = lo(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, false));
+    x = lo(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xF, 0xF, false));
+    x = lo(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xF, 0xF, false));
+    x = lo(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x140, 0xF, 0xF, false));
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = lo(r[0], r[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return lo(q[0], q[1]);
+}
 // The same max over the 4 lanes of a quad with DPP quad permutes (a VALU operand route, no LDS
 // crossbar): lane l reads lane l ^ 2 (quad_perm [2,3,0,1]), then l ^ 1 ([1,0,3,2]). The max of the
 // same four values in any order is the same float.

@@ -167,6 +167,26 @@ def test_bf16_gemv(gpu, O, nr):
     assert (idx == np.argmax(yy, axis=1)).all()
 
 
+@pytest.mark.parametrize("n,off", [(1, 0), (3, 0), (4, 0), (4099, 0), (62080, 0), (40001, 1)])
+def test_argmax_rows_edges(gpu, O, n, off):
+    """Ties across threads and waves, zeros of both signs, rows without a finite value, widths with a remainder and
+    rows that 16-byte loads cannot take."""
+    X = gpu
+    rng = np.random.default_rng(n)
+    y = rng.integers(-3, 4, (4, n)).astype(np.float32)                # many ties
+    y[1] = np.where(rng.random(n) < 0.5, np.float32(-0.0), np.float32(0.0))
+    y[2] = np.where(rng.random(n) < 0.5, np.float32(np.nan), np.float32(np.inf))
+    y[3, : n - 1] = -np.inf
+    dl = dev(X, np.concatenate([np.zeros(off, np.float32), y.ravel()]))
+    di, dv = X.DevBuf(16), X.DevBuf(16)
+    X.call("q27x_argmax_rows", dl.ptr + 4 * off, n, n, 4, di.ptr, dv.ptr, None)
+    X.call("q27x_device_sync")
+    i_o, v_o = np.empty(4, np.int32), np.empty(4, np.float32)
+    O.lib().q27o_argmax_rows(y.ctypes.data, n, n, 4, i_o.ctypes.data, v_o.ctypes.data)
+    same("argmax", di.download(np.int32, (4,)), i_o)
+    same("value", dv.download(np.float32, (4,)), v_o)
+
+
 @pytest.mark.parametrize("x_bf16,quant_bf16", [(1, 1), (0, 0), (0, 1)])
 def test_rmsnorm_quant(gpu, O, x_bf16, quant_bf16):
     X = gpu
