@@ -262,9 +262,12 @@ __global__ __launch_bounds__(kNT) void k_gdn(GdnArgs a, int nr) {
 // Prefill scan: the same per-row arithmetic as k_gdn over all nrows rows of a chunk, with the
 // value columns spread over waves instead of the key rows over a block. Value columns of the
 // delta rule are independent given the row's (k^, q^, beta, decay), so a wave owns 16 of them:
-// lane 16 g + c holds key rows 32g..32g+31 of column c, and the four key groups' partial sums
-// S^T k, S^T q meet by lane swaps in the order ((p0 + p1) + p2) + p3, which is k_gdn's order. No
-// barrier per row: a block (WPB waves, 16 WPB columns of one head) only synchronises per batch
+// lane 4 c + g holds key rows 32g..32g+31 of column c, and the four key groups' partial sums
+// S^T k, S^T q meet in their quad by DPP broadcasts in the order ((p0 + p1) + p2) + p3, which is
+// k_gdn's order (groups on 16-lane rows, meeting by lane swaps, put ~20 more dependent instructions
+// into every row: 519 against 484 us per 1024 rows). Bound by the issue of a row's ~165 instructions,
+// 128 of them the fmaf chains and the state update, on one wave per SIMD (two waves per SIMD on half
+// the CUs: 715 us). No barrier per row: a block (WPB waves, 16 WPB columns of one head) only synchronises per batch
 // of staged rows, to share the q/k norms. The state stays in registers from the first row to the
 // last and is written back once. Each row's mixed values go to `mix` [nrows][vh*128] fp32;
 // k_gdn_gnorm applies the gated RMSNorm afterwards (it needs the head's 128 columns, which live in
@@ -300,24 +303,9 @@ __global__ __launch_bounds__(256) void k_gdn_qknorm(const uint16_t* __restrict__
 #define Q27X_SCAN_WPB 4
 #endif
 constexpr int kScanWPB = Q27X_SCAN_WPB;  // waves per block
-// ((p0 + p1) + p2) + p3 over the lanes c, 16 + c, 32 + c, 48 + c (p_g in lane 16 g + c), exact in
-// the lanes of group 0 (the other lanes hold partial values). The gfx950 lane swaps exchange
-// 16-lane rows 0<->1, 2<->3 and the 32-lane halves; the second result holds the partner's value
-// in the even rows / lower half.
-__device__ __forceinline__ float key_group_sum_g0(float x) {
-    const float a = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
-    const float b = __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[1]);
-    const float c = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(b), __float_as_uint(b), false, false)[1]);
-    return ((x + a) + b) + c;      // group 0: a = p1, b = p2, c = p3 (row 1's b is row 3's x)
-}
-// group 0's value in every lane of its column: row 0 -> row 1 by a 16-lane swap, rows 0, 1 -> rows
-// 2, 3 by a 32-lane swap (the first result holds the partner's value in the odd rows / upper half)
-__device__ __forceinline__ float from_group0(float s) {
-    const int g = (threadIdx.x >> 4) & 3;
-    const float t = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false)[0]);
-    const float u = (g == 1) ? t : s;
-    const float w = __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(u), __float_as_uint(u), false, false)[0]);
-    return (g >= 2) ? w : u;
+// ((p0 + p1) + p2) + p3 of a quad of lanes (p_g in lane g), in all four lanes, by DPP quad broadcasts
+__device__ __forceinline__ float quad_sum(float x) {
+    return ((quad_bcast(x, 0) + quad_bcast(x, 1)) + quad_bcast(x, 2)) + quad_bcast(x, 3);
 }
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_gdn_scan(GdnArgs a, const float* __restrict__ qk,
@@ -330,7 +318,7 @@ __global__ __launch_bounds__(64 * WPB) void k_gdn_scan(GdnArgs a, const float* _
     static_assert(CPT >= 1 && CPT * NT == 2 * kD && BPH * NC == kD, "1, 2 or 4 waves per block");
     const int h = blockIdx.x / BPH, part = blockIdx.x % BPH;
     const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int g = lane >> 4, cw = 16 * wv + (lane & 15);      // column within the block's NC
+    const int g = lane & 3, cw = 16 * wv + (lane >> 2);       // column within the block's NC
     const int col = NC * part + cw;
     const int ratio = a.vh / a.kh, kk = h / ratio;
     const int KD = a.kh * kD;
@@ -405,11 +393,11 @@ __global__ __launch_bounds__(64 * WPB) void k_gdn_scan(GdnArgs a, const float* _
                 accA = __builtin_fmaf(st[j], r.k[j], accA);
                 accB = __builtin_fmaf(st[j], r.q[j], accB);
             }
-            const float A = from_group0(key_group_sum_g0(accA));
+            const float A = quad_sum(accA);
             const float delta = (r.v - r.decay * A) * r.beta;
 #pragma unroll
             for (int j = 0; j < kJ; ++j) st[j] = __builtin_fmaf(r.k[j], delta, r.decay * st[j]);
-            const float B = key_group_sum_g0(accB);                 // needed in group 0 only
+            const float B = quad_sum(accB);
             const float mixed = __builtin_fmaf(delta, r.kq, r.decay * B);
             if (g == 0) smix[n][cw] = mixed;
         };
