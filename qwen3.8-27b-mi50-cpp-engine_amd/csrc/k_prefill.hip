@@ -130,14 +130,19 @@ int launch_pf_conv(const uint16_t* buf, int ld, int C, int nconv, const uint16_t
 // decode path's order: 8-element chunk c on lane c % 64 in ascending c, fmaf per element, the
 // shfl tree, bf16 rounding; k_bf16_gemv2_tile, src/q27_util.hip:114-167), then
 // decay = exp(-exp(A_log) softplus(a + dt_bias)) and beta = sigmoid(b) (src/q27_gdn.hip:206-372)
-// into out [2][C][vh]. A block stages kAbTok rows y in LDS; each wave holds one weight row's
-// chunks in registers (lane l: chunks l, l + 64, ...) and runs it against every staged row.
+// into out [2][C][vh]. A block stages kAbTok rows y in LDS (bf16); each of its 8 waves holds the
+// chunks of two weight rows in registers as fp32 (lane l: chunks l, l + 64, ...) and runs both
+// against every staged row, so a staged value is read and widened once for two rows. Bound by VALU
+// issue (3 instructions per two products; one row per wave with both operands widened at the
+// product took 6, on half the CUs): 1024 rows x 96 x 5120 92 -> 76 us
+// beside another chunk's scan, which holds 96 CUs.
 constexpr int kAbTok = 8;            // rows per block
+constexpr int kAbWaves = 8;          // waves per block, two weight rows each
 constexpr int kAbChunks = 10;        // weight chunks per lane at most (K <= 5120)
 // KC: chunks per lane (every lane runs KC of them; chunks past K / 8 have zero weights, and
 // fma(0, x, acc) = acc for the finite normed rows, so they change nothing)
 template <int KC>
-__global__ __launch_bounds__(1024) void k_pf_ab(const uint16_t* __restrict__ in_a, const uint16_t* __restrict__ in_b,
+__global__ __launch_bounds__(64 * kAbWaves) void k_pf_ab(const uint16_t* __restrict__ in_a, const uint16_t* __restrict__ in_b,
                                                 const uint16_t* __restrict__ A_log,
                                                 const uint16_t* __restrict__ dt_bias, const uint16_t* __restrict__ y,
                                                 int ystride, int K, int vh, int C, float* __restrict__ out) {
@@ -145,44 +150,61 @@ __global__ __launch_bounds__(1024) void k_pf_ab(const uint16_t* __restrict__ in_
     const int t0 = blockIdx.x * kAbTok, nt = (C - t0 < kAbTok) ? C - t0 : kAbTok;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nch = K >> 3;
-    for (int i = threadIdx.x; i < nt * nch; i += 1024) {
+    for (int i = threadIdx.x; i < nt * nch; i += 64 * kAbWaves) {
         const int n = i / nch, c = i - n * nch;
         sy[i] = *(const uint4*)(y + (size_t)(t0 + n) * ystride + 8 * c);
     }
-    __syncthreads();
-    for (int j = wv; j < 2 * vh; j += 16) {
-        const int which = j / vh, head = j - which * vh;
-        const uint16_t* wrow = (which ? in_b : in_a) + (size_t)head * K;
-        uint4 w[KC];
+    // weight rows j0, j0 + 1 of the stacked in_a | in_b (2 vh rows: always whole pairs)
+    const int j0 = 2 * (blockIdx.y * kAbWaves + wv);
+    float w[2][KC][8];
+    if (j0 < 2 * vh) {
 #pragma unroll
-        for (int i = 0; i < KC; ++i) {
-            const int c = lane + 64 * i;
-            w[i] = *(const uint4*)(wrow + 8 * (c < nch ? c : 0));
-            if (c >= nch) w[i] = make_uint4(0u, 0u, 0u, 0u);
-        }
-        const float Aexp = which ? 0.0f : qexp(bf2f(A_log[head]));
-        const float dtb = which ? 0.0f : bf2f(dt_bias[head]);
-        for (int n = 0; n < nt; ++n) {
-            const uint4* yr = sy + (size_t)n * nch;
-            float acc = 0.0f;
+        for (int r = 0; r < 2; ++r) {
+            const int j = j0 + r;
+            const uint16_t* wrow = j < vh ? in_a + (size_t)j * K : in_b + (size_t)(j - vh) * K;
 #pragma unroll
             for (int i = 0; i < KC; ++i) {
                 const int c = lane + 64 * i;
-                const uint4 x = yr[c < nch ? c : 0];
-                acc = __builtin_fmaf(__uint_as_float(w[i].x << 16), __uint_as_float(x.x << 16), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].x & 0xFFFF0000u), __uint_as_float(x.x & 0xFFFF0000u), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].y << 16), __uint_as_float(x.y << 16), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].y & 0xFFFF0000u), __uint_as_float(x.y & 0xFFFF0000u), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].z << 16), __uint_as_float(x.z << 16), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].z & 0xFFFF0000u), __uint_as_float(x.z & 0xFFFF0000u), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].w << 16), __uint_as_float(x.w << 16), acc);
-                acc = __builtin_fmaf(__uint_as_float(w[i].w & 0xFFFF0000u), __uint_as_float(x.w & 0xFFFF0000u), acc);
+                uint4 v = *(const uint4*)(wrow + 8 * (c < nch ? c : 0));
+                if (c >= nch) v = make_uint4(0u, 0u, 0u, 0u);
+                const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    w[r][i][2 * e] = __uint_as_float(u[e] << 16);
+                    w[r][i][2 * e + 1] = __uint_as_float(u[e] & 0xFFFF0000u);
+                }
             }
-            const float v = bfr(bcast0(tree64(acc)));
-            if (lane == 0) {
-                const float r = which ? qsigmoid(v) : qexp(-(Aexp * qsoftplus(v + dtb)));
-                out[((size_t)which * C + t0 + n) * vh + head] = r;
+        }
+    }
+    __syncthreads();
+    if (j0 >= 2 * vh) return;
+    // lanes 0 and 1 turn the two rows' logits into decay = exp(-exp(A_log) softplus(a + dt)) or beta = sigmoid(b)
+    const int j = j0 + (lane & 1), which = j >= vh, head = j - which * vh;
+    const float Aexp = which ? 0.0f : qexp(bf2f(A_log[head]));
+    const float dtb = which ? 0.0f : bf2f(dt_bias[head]);
+    for (int n = 0; n < nt; ++n) {
+        const uint4* yr = sy + (size_t)n * nch;
+        float acc[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            const int c = lane + 64 * i;
+            const uint4 x = yr[c < nch ? c : 0];
+            const uint32_t u[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float lo = __uint_as_float(u[e] << 16), hi = __uint_as_float(u[e] & 0xFFFF0000u);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    acc[r] = __builtin_fmaf(w[r][i][2 * e], lo, acc[r]);
+                    acc[r] = __builtin_fmaf(w[r][i][2 * e + 1], hi, acc[r]);
+                }
             }
+        }
+        const float a0 = bcast0(tree64(acc[0])), a1 = bcast0(tree64(acc[1]));
+        const float v = bfr((lane & 1) ? a1 : a0);
+        if (lane < 2) {
+            const float r = which ? qsigmoid(v) : qexp(-(Aexp * qsoftplus(v + dtb)));
+            out[((size_t)which * C + t0 + n) * vh + head] = r;
         }
     }
 }
@@ -204,11 +226,11 @@ int launch_pf_ab(const uint16_t* in_a, const uint16_t* in_b, const uint16_t* A_l
         lds_set = true;
     }
     const int kc = (K / 8 + 63) / 64;
-    const dim3 grid((unsigned)((C + kAbTok - 1) / kAbTok));
-    if (kc <= 2) hipLaunchKernelGGL(k_pf_ab<2>, grid, dim3(1024), lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else if (kc <= 4) hipLaunchKernelGGL(k_pf_ab<4>, grid, dim3(1024), lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else if (kc <= 8) hipLaunchKernelGGL(k_pf_ab<8>, grid, dim3(1024), lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else hipLaunchKernelGGL(k_pf_ab<10>, grid, dim3(1024), lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
+    const dim3 grid((unsigned)((C + kAbTok - 1) / kAbTok), (unsigned)((vh + kAbWaves - 1) / kAbWaves)), blk(64 * kAbWaves);
+    if (kc <= 2) hipLaunchKernelGGL(k_pf_ab<2>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
+    else if (kc <= 4) hipLaunchKernelGGL(k_pf_ab<4>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
+    else if (kc <= 8) hipLaunchKernelGGL(k_pf_ab<8>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
+    else hipLaunchKernelGGL(k_pf_ab<10>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }
