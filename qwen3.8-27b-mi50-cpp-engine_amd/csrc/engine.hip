@@ -1406,12 +1406,16 @@ static int pf_attn_rows(const q27x_config& c, int max_splits, int pos, int left)
     return n;
 }
 static int env_int(const char* name, int def);
-// Rows per pass over the layers for an n-token prompt: 1024 from 2048 tokens on, else 512 (with the two
-// streams below, smaller chunks overlap more: at 4096 tokens 1024-row chunks measured 15.1K tok/s
-// against 14.0K with 2048 and 11.3K with one stream; 512 and 768 were slower). Q27X_PF_CHUNK
-// (8 .. 4096) overrides, read per call.
+// Rows per pass over the layers for an n-token prompt: up to 512 tokens one chunk, else an even
+// number of equal chunks of at most 2048 rows (whole 64s). Chunks run in pairs on the two streams
+// below, one's GDN scan beside the other's GEMMs: an odd last chunk runs alone, and a short one
+// leaves its partner alone. 16 layers, ms, 512-row chunks below 2048 tokens and 1024-row ones from
+// there / now: 600 tokens 11.6 / 11.0, 1300 21.9 / 18.3, 2600 40.0 / 37.1, 3300 51.8 / 49.5, 5000
+// 82.7 / 78.4, 8000 147.4 / 144.2; 300 tokens in two chunks 2.6 against 2.2 (4 layers).
+// Q27X_PF_CHUNK (8 .. 4096) overrides, read per call.
 static int pf_chunk(int n) {
-    const int v = env_int("Q27X_PF_CHUNK", n >= 2048 ? 1024 : 512);
+    const int k = n <= 512 ? 1 : 2 * ((n + 4095) / 4096);
+    const int v = env_int("Q27X_PF_CHUNK", n <= 512 ? 512 : ((n + k - 1) / k + 63) / 64 * 64);
     return v < 8 ? 8 : (v > 4096 ? 4096 : v);
 }
 // successive chunks on two streams, chunk c + 1's layer l behind chunk c's layer l (Q27X_PF_PIPE=0: one
