@@ -262,19 +262,26 @@ __global__ __launch_bounds__(kNT) void k_gdn(GdnArgs a, int nr) {
 // Prefill scan: the same per-row arithmetic as k_gdn over all nrows rows of a chunk, with the
 // value columns spread over waves instead of the key rows over a block. Value columns of the
 // delta rule are independent given the row's (k^, q^, beta, decay), so a wave owns 16 of them:
-// lane 4 c + g holds key rows 32g..32g+31 of column c, and the four key groups' partial sums
-// S^T k, S^T q meet in their quad by DPP broadcasts in the order ((p0 + p1) + p2) + p3, which is
-// k_gdn's order (groups on 16-lane rows, meeting by lane swaps, put ~20 more dependent instructions
-// into every row: 519 against 484 us per 1024 rows). Bound by the issue of a row's ~165 instructions,
-// 128 of them the fmaf chains and the state update, on one wave per SIMD (two waves per SIMD on half
-// the CUs: 715 us). No barrier per row: a block (WPB waves, 16 WPB columns of one head) only synchronises per batch
-// of staged rows, to share the q/k norms. The state stays in registers from the first row to the
-// last and is written back once. Each row's mixed values go to `mix` [nrows][vh*128] fp32;
-// k_gdn_gnorm applies the gated RMSNorm afterwards (it needs the head's 128 columns, which live in
-// several blocks). Row scalars: decay at rowsc[n vh + h], beta at rowsc[(nrows + n) vh + h].
+// lane 16 g + c holds key rows 32g..32g+31 of column c. S^T k and S^T q are two chains of 32
+// products per lane; a lane holds two of its group's k^ and q^ values and the products take the
+// others from the 16-lane row by the instruction's broadcast operand, so that a row is one 16-byte
+// LDS read per lane. The four key groups' partial sums meet in the order ((p0 + p1) + p2) + p3 by
+// lane swaps. The update S = k^ delta + decay S runs on the matrix cores in the 4x4x1 fp32 form (16
+// independent 4x4 blocks, 4 key rows a step, one fused multiply-add per element: the same bits as
+// k_gdn's fmaf, subnormals included), k^ again from the same registers by the instruction's A
+// broadcast. The state stays in registers from the first row to the last and is written back once.
+// Rows are staged by LDS DMA in three batches. Bound by one wave's instructions per SIMD (~145 a
+// row). Per 300 rows of 48 heads: 150 us with quads of lanes holding a column's groups, the row in
+// 16 LDS reads whose groups met in the same banks, and staging through registers; 124 with those
+// reads free of conflicts and the DMA staging; 110 as here. (S^T k and S^T q on the matrix cores as
+// well, as rows 0 and 1 of one chain of 32 steps: 141, a dependent step takes ~28 clocks.)
+// Each row's mixed values go to `mix` [nrows][vh*128] fp32; k_gdn_gnorm applies the gated RMSNorm
+// afterwards (it needs the head's 128 columns, which live in two blocks). Row scalars: decay at
+// rowsc[n vh + h], beta at rowsc[(nrows + n) vh + h].
 // q/k norms of the scan's rows, outside the scan (they do not depend on the state): one wave per
 // (row, key head), k_gdn's arithmetic (two 64-lane trees per sum, first half + second half).
-// qk [nrows][kh][256]: q^ (128) then k^ (128); kq [nrows][kh]: k^.q^.
+// qk [nrows][kh][4][16][4]: at [g][c] the key rows 32 g + c and 32 g + 16 + c of k^, then of q^ (the
+// scan's lane 16 g + c reads them at once). kq [nrows][kh]: k^.q^.
 __global__ __launch_bounds__(256) void k_gdn_qknorm(const uint16_t* __restrict__ qkv, int qkv_stride, int kh,
                                                     int nrows, float* __restrict__ qk, float* __restrict__ kq) {
     const int lane = threadIdx.x & 63;
@@ -292,133 +299,185 @@ __global__ __launch_bounds__(256) void k_gdn_qknorm(const uint16_t* __restrict__
     const float ssk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sk0 + sk1)));
     const float invq = rsqrt_cr(ssq + 1e-6f) * 0.0883883476f;
     const float invk = rsqrt_cr(ssk + 1e-6f);
-    float* d = qk + (size_t)u * 2 * kD;
-    d[lane] = q0 * invq;
-    d[64 + lane] = q1 * invq;
-    d[kD + lane] = k0 * invk;
-    d[kD + 64 + lane] = k1 * invk;
+    float* d = qk + (size_t)u * 2 * kD + (lane >> 5) * 64 + (lane & 15) * 4 + ((lane >> 4) & 1);
+    d[2] = q0 * invq;
+    d[128 + 2] = q1 * invq;          // key row 64 + lane: two groups on
+    d[0] = k0 * invk;
+    d[128] = k1 * invk;
     if (lane == 0) kq[u] = ((sx0 + sx1) * invq) * invk;
 }
-#ifndef Q27X_SCAN_WPB
-#define Q27X_SCAN_WPB 4
-#endif
-constexpr int kScanWPB = Q27X_SCAN_WPB;  // waves per block
-// ((p0 + p1) + p2) + p3 of a quad of lanes (p_g in lane g), in all four lanes, by DPP quad broadcasts
-__device__ __forceinline__ float quad_sum(float x) {
-    return ((quad_bcast(x, 0) + quad_bcast(x, 1)) + quad_bcast(x, 2)) + quad_bcast(x, 3);
+constexpr int kScanW = 4;                    // waves per block, 16 value columns each
+constexpr int kScanR = 16;                   // rows staged per batch, three batches in LDS
+constexpr int kScanNC = 16 * kScanW;         // value columns of a block
+typedef float v4f __attribute__((ext_vector_type(4)));
+// c + a b per element of 16 4x4 blocks: lane 4 blk + i holds a's row i, b's column i and c's column
+// i (registers are c's rows); blocks 4 n .. 4 n + 3 all take a from block 4 n + M
+template <int M>
+__device__ __forceinline__ v4f mfma4(float a, float b, const v4f& c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 2, M, 0);
 }
-template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void k_gdn_scan(GdnArgs a, const float* __restrict__ qk,
-                                                      const float* __restrict__ kqv, float* __restrict__ mix,
-                                                      int nrows) {
-    constexpr int NT = 64 * WPB, NC = 16 * WPB;          // threads, value columns of the block
-    constexpr int R = 8 * WPB;                           // rows staged per batch
-    constexpr int CPT = 2 * kD / NT;                     // q|k channels loaded per thread
-    constexpr int BPH = kD / NC;                         // blocks per head
-    static_assert(CPT >= 1 && CPT * NT == 2 * kD && BPH * NC == kD, "1, 2 or 4 waves per block");
+// a = fma(k of lane n of the 16-lane row, s[n], a) over n = 0..15 in order, and b the same from q: two
+// chains side by side, the broadcast part of each instruction (the compiler makes it a move of its
+// own). One block, because the hardware leaves two waits to the program: a lane-broadcast operand
+// must not be written by the two instructions before, nor a VALU operand by a matrix instruction
+// less than five before.
+__device__ __forceinline__ void chain16(float& a, float& b, float k, float q, const v4f& s0, const v4f& s1,
+                                        const v4f& s2, const v4f& s3) {
+#define Q27X_STEP(S, N) "v_fmac_f32_dpp %0, %2, " S " row_newbcast:" N " row_mask:0xf bank_mask:0xf\n\t" \
+                        "v_fmac_f32_dpp %1, %3, " S " row_newbcast:" N " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 4\n\t"
+                 Q27X_STEP("%4", "0")
+                 Q27X_STEP("%5", "1")
+                 Q27X_STEP("%6", "2")
+                 Q27X_STEP("%7", "3")
+                 Q27X_STEP("%8", "4")
+                 Q27X_STEP("%9", "5")
+                 Q27X_STEP("%10", "6")
+                 Q27X_STEP("%11", "7")
+                 Q27X_STEP("%12", "8")
+                 Q27X_STEP("%13", "9")
+                 Q27X_STEP("%14", "10")
+                 Q27X_STEP("%15", "11")
+                 Q27X_STEP("%16", "12")
+                 Q27X_STEP("%17", "13")
+                 Q27X_STEP("%18", "14")
+                 Q27X_STEP("%19", "15")
+                 : "+v"(a), "+v"(b)
+                 : "v"(k), "v"(q), "v"(s0[0]), "v"(s0[1]), "v"(s0[2]), "v"(s0[3]), "v"(s1[0]), "v"(s1[1]),
+                   "v"(s1[2]), "v"(s1[3]), "v"(s2[0]), "v"(s2[1]), "v"(s2[2]), "v"(s2[3]), "v"(s3[0]), "v"(s3[1]),
+                   "v"(s3[2]), "v"(s3[3]));
+#undef Q27X_STEP
+}
+// odd 16-lane rows of x change places with the even rows of y; the upper half of x with y's lower
+__device__ __forceinline__ void lane_swap16(float& x, float& y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]); y = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void lane_swap32(float& x, float& y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]); y = __uint_as_float(r[1]);
+}
+// ((p0 + p1) + p2) + p3 of lanes c, 16 + c, 32 + c, 48 + c, in all four
+__device__ __forceinline__ float row_sum4(float x) {
+    float p0 = x, p1 = x;
+    lane_swap16(p0, p1);                 // rows p0 p0 p2 p2, p1 p1 p3 p3
+    float p2 = p0, p3 = p1;
+    lane_swap32(p0, p2);
+    lane_swap32(p1, p3);
+    return ((p0 + p1) + p2) + p3;
+}
+__global__ __launch_bounds__(64 * kScanW, 2) void k_gdn_scan(GdnArgs a, const float* __restrict__ qk,
+                                                         const float* __restrict__ kqv, float* __restrict__ mix,
+                                                         int nrows) {
+    constexpr int R = kScanR, NC = kScanNC, BPH = kD / NC;
+    constexpr int NS = 3 * R;                              // row slots in LDS, row n in slot n % NS
+    static_assert(R % 8 == 0 && R >= 16 && R <= 64 && NC == 64, "whole DMA instructions per batch");
     const int h = blockIdx.x / BPH, part = blockIdx.x % BPH;
     const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int g = lane & 3, cw = 16 * wv + (lane >> 2);       // column within the block's NC
+    const int g = lane >> 4, cw = 16 * wv + (lane & 15);      // column within the block's NC
     const int col = NC * part + cw;
     const int ratio = a.vh / a.kh, kk = h / ratio;
-    const int KD = a.kh * kD;
     const size_t mstride = (size_t)a.vh * kD;
-    __shared__ float sv[R][NC];                  // v of the block's columns
-    __shared__ __attribute__((aligned(16))) float sq[R][kD];
-    __shared__ __attribute__((aligned(16))) float sk[R][kD];
-    __shared__ float srow[R][4];                 // per row: kq, beta, decay
-    __shared__ float smix[R][NC];
+    __shared__ __attribute__((aligned(1024))) float sqk[NS][2 * kD];   // k^, q^ as k_gdn_qknorm lays them out
+    __shared__ __attribute__((aligned(256))) uint16_t sv[NS][NC];      // v of the block's columns
+    __shared__ __attribute__((aligned(256))) float ssc[3][NS];         // decay, beta, k^.q^
     float* Sp = a.S + (size_t)h * kD * kD + (size_t)(g * kJ) * kD + col;
-    float st[kJ];
+    v4f st[kJ / 4];                                           // st[r][m]: key row 32 g + 4 r + m
 #pragma unroll
-    for (int j = 0; j < kJ; ++j) st[j] = Sp[(size_t)j * kD];
-    // thread t loads the normed q^|k^ values t + NT i of the key head (< 128: q^, else k^) and v
-    // column NC part + t % NC
-    const size_t chv = (size_t)2 * KD + (size_t)h * kD + NC * part + (t % NC);
-    float xr[R][CPT];
-    uint16_t xv[R];
-    float r_a = 0.0f, r_b = 0.0f, r_kq = 0.0f;
-    // unconditional loads (rows past the last repeat it; every thread loads a v column): a load
-    // under a condition is followed by its own wait, which would serialise the batch's loads
-    auto load = [&](int r0) {
+    for (int j = 0; j < kJ; ++j) st[j >> 2][j & 3] = Sp[(size_t)j * kD];
+    const uint32_t lqk = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&sqk[0][0];
+    const uint32_t lv = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&sv[0][0];
+    const uint32_t lsc = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&ssc[0][0];
+    const uint16_t* vsrc = a.qkv + (size_t)2 * a.kh * kD + (size_t)h * kD + NC * part;
+    // batch b by LDS DMA: wave wv brings rows wv, wv + 4, ... (1 KiB of k^ and q^ each), every
+    // fourth pair of v rows (32 lanes of 4 bytes a row), and waves 0..2 one of the row scalars.
+    // Rows past the last repeat it.
+    auto load = [&](int b) {
+        const int r0 = b * R, s0 = (b % 3) * R;
 #pragma unroll
-        for (int n = 0; n < R; ++n) {
-            const int rn = (r0 + n < nrows) ? r0 + n : nrows - 1;
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) xr[n][i] = qk[((size_t)rn * a.kh + kk) * 2 * kD + t + NT * i];
-            xv[n] = a.qkv[(size_t)rn * a.qkv_stride + chv];
+        for (int i = 0; i < R / kScanW; ++i) {
+            const int n = wv + kScanW * i, rn = (r0 + n < nrows) ? r0 + n : nrows - 1;
+            lds_dma16_at(qk + ((size_t)rn * a.kh + kk) * 2 * kD, 16 * lane, lqk + (s0 + n) * (2 * kD * 4));
         }
-        const int rt = (r0 + (t % R) < nrows) ? r0 + (t % R) : nrows - 1;
-        r_a = a.rowsc[(size_t)rt * a.vh + h];
-        r_b = a.rowsc[(size_t)(nrows + rt) * a.vh + h];
-        r_kq = kqv[(size_t)rt * a.kh + kk];
+#pragma unroll
+        for (int i = 0; i < R / 2 / kScanW; ++i) {
+            const int n = 2 * (wv + kScanW * i);
+            const int m = r0 + n + (lane >> 5), rn = (m < nrows) ? m : nrows - 1;
+            lds_dma4(vsrc + (size_t)rn * a.qkv_stride + 2 * (lane & 31), lv + (s0 + n) * (NC * 2));
+        }
+        if (wv < 3 && lane < R) {
+            const int rn = (r0 + lane < nrows) ? r0 + lane : nrows - 1;
+            const float* p = (wv == 2) ? kqv + (size_t)rn * a.kh + kk
+                                       : a.rowsc + (size_t)(wv * nrows + rn) * a.vh + h;
+            lds_dma4(p, lsc + (wv * NS + s0) * 4);
+        }
     };
+    // a row's operands: k^ (x, y) and q^ (z, w) of key rows 32 g + (lane & 15) and + 16
+    struct RowIn { float4 kq4; float decay, beta, kq; uint16_t v; };
+    auto lds_row = [&](int s, RowIn& r) {
+        r.kq4 = *(const float4*)&sqk[s][4 * lane];
+        r.decay = ssc[0][s]; r.beta = ssc[1][s]; r.kq = ssc[2][s]; r.v = sv[s][cw];
+    };
+    float keep = 0.0f;
+    // One row; what the next one (slot sn) reads from LDS is requested here. Lanes g == u keep its
+    // mixed value.
+    auto do_row = [&](const RowIn& r, RowIn& x, int sn, int u) {
+        lds_row(sn, x);
+        float accA = 0.0f, accB = 0.0f;
+        chain16(accA, accB, r.kq4.x, r.kq4.z, st[0], st[1], st[2], st[3]);
+        chain16(accA, accB, r.kq4.y, r.kq4.w, st[4], st[5], st[6], st[7]);
+        v4f ds[kJ / 4];
+#pragma unroll
+        for (int i = 0; i < kJ / 4; ++i) ds[i] = r.decay * st[i];
+        const float A = row_sum4(accA);
+        const float delta = (bf2f(r.v) - r.decay * A) * r.beta;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const float ku = n ? r.kq4.y : r.kq4.x;
+            st[4 * n] = mfma4<0>(ku, delta, ds[4 * n]);
+            st[4 * n + 1] = mfma4<1>(ku, delta, ds[4 * n + 1]);
+            st[4 * n + 2] = mfma4<2>(ku, delta, ds[4 * n + 2]);
+            st[4 * n + 3] = mfma4<3>(ku, delta, ds[4 * n + 3]);
+        }
+        const float B = row_sum4(accB);
+        float mixed = __builtin_fmaf(delta, r.kq, r.decay * B);
+        asm("" : "+v"(mixed));                    // computed by all lanes: no branch around it
+        keep = (g == u) ? mixed : keep;
+    };
+    float* mo = mix + (size_t)h * kD + col;
     load(0);
-    for (int r0 = 0; r0 < nrows; r0 += R) {
-        const int nr = (nrows - r0 < R) ? nrows - r0 : R;
-        __syncthreads();                            // the previous batch is written out
-        if (t < nr) { srow[t][0] = r_kq; srow[t][1] = r_b; srow[t][2] = r_a; }
-        // every staged row is written (rows past nr hold copies of the last row and are not read):
-        // an exit at nr would index the register arrays dynamically (a select chain per element)
-#pragma unroll
-        for (int n = 0; n < R; ++n) {
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) {
-                const int c = t + NT * i;
-                if (c < kD) sq[n][c] = xr[n][i];
-                else sk[n][c - kD] = xr[n][i];
-            }
-            if (t < NC) sv[n][t] = bf2f(xv[n]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (R < nrows) load(1);
+    RowIn ra, rb;
+    lds_row(0, ra);
+    const int n4 = nrows >> 2;
+    int slot = 0;                                     // of row 4 G
+    for (int G = 0; G < n4; ++G) {
+        if (G % (R / 4) == R / 4 - 1) {               // before a batch's last rows, which request the next batch's first
+            // this wave's DMAs have landed: the two operations that may stay in flight are younger
+            // mix stores (R/4 of them follow a batch's DMAs, R/4 - 1 the prologue's)
+            asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+            __syncthreads();                          // and everyone is done with the batch before this one
+            const int b = G / (R / 4) + 2;
+            if (b * R < nrows) load(b);
         }
-        if (r0 + R < nrows) load(r0 + R);            // next batch in flight during this one
-        __syncthreads();
-        // rows in pairs: everything a row reads from LDS is requested while the row before it
-        // computes (a row's own reads would make every wait cover the prefetch behind them)
-        struct RowIn { float k[kJ], q[kJ]; float kq, beta, decay, v; };
-        auto lds_row = [&](int n, RowIn& r) {
-#pragma unroll
-            for (int j4 = 0; j4 < kJ; j4 += 4) {
-                const float4 k4 = *(const float4*)&sk[n][g * kJ + j4];
-                const float4 q4 = *(const float4*)&sq[n][g * kJ + j4];
-                r.k[j4] = k4.x; r.k[j4 + 1] = k4.y; r.k[j4 + 2] = k4.z; r.k[j4 + 3] = k4.w;
-                r.q[j4] = q4.x; r.q[j4 + 1] = q4.y; r.q[j4 + 2] = q4.z; r.q[j4 + 3] = q4.w;
-            }
-            r.kq = srow[n][0]; r.beta = srow[n][1]; r.decay = srow[n][2];
-            r.v = sv[n][cw];
-        };
-        auto do_row = [&](int n, const RowIn& r) {
-            float accA = 0.0f, accB = 0.0f;
-#pragma unroll
-            for (int j = 0; j < kJ; ++j) {
-                accA = __builtin_fmaf(st[j], r.k[j], accA);
-                accB = __builtin_fmaf(st[j], r.q[j], accB);
-            }
-            const float A = quad_sum(accA);
-            const float delta = (r.v - r.decay * A) * r.beta;
-#pragma unroll
-            for (int j = 0; j < kJ; ++j) st[j] = __builtin_fmaf(r.k[j], delta, r.decay * st[j]);
-            const float B = quad_sum(accB);
-            const float mixed = __builtin_fmaf(delta, r.kq, r.decay * B);
-            if (g == 0) smix[n][cw] = mixed;
-        };
-        // (the prefetches are unconditional, of row min(n, nr - 1), so that every path through the
-        // loop has the same reads in flight and the waits count only the reads a row needs)
-        RowIn ra, rb;
-        lds_row(0, ra);
-        for (int n = 0; n < nr; n += 2) {
-            lds_row((n + 1 < nr) ? n + 1 : nr - 1, rb);
-            do_row(n, ra);
-            lds_row((n + 2 < nr) ? n + 2 : nr - 1, ra);
-            if (n + 1 < nr) do_row(n + 1, rb);
-        }
-        __syncthreads();
-        for (int i = t; i < nr * NC; i += NT) {
-            const int n = i / NC, c = i % NC;
-            mix[(size_t)(r0 + n) * mstride + (size_t)h * kD + NC * part + c] = smix[n][c];
-        }
+        do_row(ra, rb, slot + 1, 0);
+        do_row(rb, ra, slot + 2, 1);
+        do_row(ra, rb, slot + 3, 2);
+        slot = (slot + 4 == NS) ? 0 : slot + 4;
+        // (the last group's request past the end reads a row of an older batch, unused)
+        do_row(rb, ra, slot, 3);
+        mo[(size_t)(4 * G + g) * mstride] = keep;
+    }
+    for (int n = 4 * n4; n < nrows; ++n) {            // one to three last rows
+        do_row(ra, rb, slot + 1, 0);                  // (slot <= NS - 2 here)
+        if (g == 0) mo[(size_t)n * mstride] = keep;
+        ++slot;
+        ra = rb;
     }
 #pragma unroll
-    for (int j = 0; j < kJ; ++j) Sp[(size_t)j * kD] = st[j];
+    for (int j = 0; j < kJ; ++j) Sp[(size_t)j * kD] = st[j >> 2][j & 3];
 }
 // gated RMSNorm of the scan's rows (k_gdn's arithmetic: two 64-lane trees of mixed^2, their sum
 // over 128, rsqrt; y = mixed inv norm_w SiLU(z) -> bf16). One 128-thread block per (head, row).
@@ -438,15 +497,16 @@ __global__ __launch_bounds__(kD) void k_gdn_gnorm(const float* __restrict__ mix,
 }
 int launch_gdn_scan(const GdnArgs& a, int nrows, float* qk, float* kq, float* mix, hipStream_t s) {
     if (a.d != kD || a.kh < 1 || a.vh % a.kh || nrows < 1 || !a.qkv || !a.z || !a.S || !a.rowsc || !a.out ||
-        !a.norm_w || !mix || !qk || !kq || nrows > 65535) {
+        !a.norm_w || !mix || !qk || !kq || nrows > 65535 ||
+        ((uintptr_t)a.qkv & 3) || (a.qkv_stride & 1)) {
         set_error("gdn scan: unsupported shape or null argument (d=%d kh=%d vh=%d rows=%d)", a.d, a.kh, a.vh, nrows);
         return Q27X_E_SHAPE;
     }
     hipLaunchKernelGGL(k_gdn_qknorm, dim3((unsigned)((nrows * a.kh + 3) / 4)), dim3(256), 0, s, a.qkv, a.qkv_stride,
                        a.kh, nrows, qk, kq);
     Q27X_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_gdn_scan<kScanWPB>, dim3(a.vh * (kD / (16 * kScanWPB))), dim3(64 * kScanWPB), 0, s, a,
-                       (const float*)qk, (const float*)kq, mix, nrows);
+    hipLaunchKernelGGL(k_gdn_scan, dim3(a.vh * (kD / kScanNC)), dim3(64 * kScanW), 0, s, a, (const float*)qk,
+                       (const float*)kq, mix, nrows);
     Q27X_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_gdn_gnorm, dim3(a.vh, nrows), dim3(kD), 0, s, (const float*)mix, a.z, a.z_stride, a.norm_w,
                        a.eps, a.vh, a.out, a.out_stride);

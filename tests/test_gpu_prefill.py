@@ -78,6 +78,13 @@ def test_tiny_prefill_gemm_forms_match_oracle(gpu, O, monkeypatch, form, gs):
     run_case(gpu, O, gpu.tiny_config(spec_k=2, pf_gs=gs), 150, 2, None)
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 31, 32, 35, 47, 48, 50, 67])
+def test_tiny_prefill_scan_row_edges_match_oracle(gpu, O, n):
+    """The GDN scan's rows around its groups of 4, its staged batches of 16 and the wrap of its three batches in
+    LDS (48 rows): state and conv history after the prompt, bit for bit."""
+    run_case(gpu, O, gpu.tiny_config(spec_k=2), n, 1)
+
+
 def test_tiny_wide_group_swiglu_prefill_matches_oracle(gpu, O):
     """inter 5120 with whole-K groups: the down projection's input is quantized per (token, 5120)
     by the wide-group SwiGLU kernel (values held in registers: 1280 quads on 1024 threads, the
