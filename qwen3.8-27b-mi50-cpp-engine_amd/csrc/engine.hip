@@ -100,7 +100,7 @@ struct PfBuf {
     float* x = nullptr;          // [cap][H] fp32 residual
     uint16_t* h = nullptr;       // [cap][H] bf16 residual copy (the next add's residual)
     uint16_t* y = nullptr;       // [cap][H] bf16 normed rows (GDN a/b)
-    float* yf = nullptr;         // [cap][H] normed values to quantize; the GDN scan's q^|k^ ([cap][kh][256])
+    float* qk = nullptr;         // the GDN scan's q^|k^ ([cap][kh][256])
     int8_t* xq = nullptr; float* xs = nullptr;     // [cap][kmax] codes, [cap][32] group scales
     int8_t* xq2 = nullptr; float* xs2 = nullptr;   // [cap][H], [cap][32]: the MTP pass's second fc input
     uint16_t* pb = nullptr;      // [cap][wmax] projection rows
@@ -1454,7 +1454,7 @@ static int pf_alloc(q27x_ctx* x, int cap, PfBuf** slot) {
     const size_t ms = (size_t)x->max_splits;
     int rc = 0;
     if ((rc = A((void**)&B->x, C * H * 4)) || (rc = A((void**)&B->h, C * H * 2)) || (rc = A((void**)&B->y, C * H * 2)) ||
-        (rc = A((void**)&B->yf, C * std::max(H, 2 * c.gdn_kh * x->D) * 4)) || (rc = A((void**)&B->xq, C * kmax)) || (rc = A((void**)&B->xs, C * 32 * 4)) ||
+        (rc = A((void**)&B->qk, C * 2 * c.gdn_kh * x->D * 4)) || (rc = A((void**)&B->xq, C * kmax)) || (rc = A((void**)&B->xs, C * 32 * 4)) ||
         (rc = A((void**)&B->xq2, C * H)) || (rc = A((void**)&B->xs2, C * 32 * 4)) ||
         (rc = A((void**)&B->pb, C * wmax * 2)) || (rc = A((void**)&B->qh, C * std::max(x->att, 1) * 2)) ||
         (rc = A((void**)&B->gu, C * std::max(2 * I, x->nz) * 4)) || (rc = A((void**)&B->mix, C * std::max(x->nz, x->att) * 2)) ||
@@ -1517,13 +1517,10 @@ static int pf_weights(q27x_ctx* x) {
     x->pf_wready = 1;
     return Q27X_OK;
 }
-// norm of C rows (values to B.yf) and their per-(token, group) codes in groups of gs columns
+// norm of C rows and their per-(token, group) codes in groups of gs columns
 static int pf_norm_quant(q27x_ctx* x, NormArgs n, int C, int8_t* xq, float* xs, int gs, float in_scale = 1.0f) {
-    PfBuf& B = *x->pfc;
-    n.yf = B.yf; n.yfstride = x->H;
-    int rc = launch_norm(n, C, x->pfs);
-    if (rc) return rc;
-    return launch_quant_tok_grp(B.yf, x->H, C, x->H, gs, in_scale, xq, xs, x->pfs);
+    n.xq = xq; n.xs = xs; n.in_scale = in_scale;
+    return launch_norm_grp(n, C, gs, x->pfs);
 }
 
 static int pf_layer(q27x_ctx* x, int l, int p0, int C) {
@@ -1574,9 +1571,8 @@ static int pf_layer(q27x_ctx* x, int l, int p0, int C) {
         g.rowsc = B.rowsc; g.norm_w = Y.gdn_norm; g.S = Y.S;
         g.kh = c.gdn_kh; g.vh = c.gdn_vh; g.d = x->D; g.eps = c.rms_eps;
         g.out = B.mix; g.out_stride = x->nz; g.stop = &d->stop;
-        // scratch: yf (free after the in_qkv|in_z GEMM's quantizer) for q^|k^, the third rowsc
-        // slab for k^.q^, the gate|up output (free until the MLP) for the mixed rows
-        if ((rc = launch_gdn_scan(g, C, B.yf, B.rowsc + (size_t)2 * B.cap * c.gdn_vh, B.gu, s))) return rc;
+        // scratch: qk for q^|k^, the third rowsc slab for k^.q^, the gate|up output (free until the MLP) for the mixed rows
+        if ((rc = launch_gdn_scan(g, C, B.qk, B.rowsc + (size_t)2 * B.cap * c.gdn_vh, B.gu, s))) return rc;
         if ((rc = launch_pf_quant_bf16(B.mix, x->nz, C, x->nz, pf_gs(c, x->nz), Y.in_s_out, B.xq, B.xs, s))) return rc;
         if ((rc = pf_gemm(x, Y.out_proj, 0, H, B.xq, B.xs, C, B.x, H, 0, B.h))) return rc;
     }

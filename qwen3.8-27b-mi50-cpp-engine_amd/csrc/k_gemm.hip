@@ -923,13 +923,13 @@ __global__ __launch_bounds__(256) void k_i8g64_to_grp(const int8_t* w, const flo
 // now 27. NV = 0: groups wider than 20480, in two passes.
 template <int T, int NV>
 __global__ __launch_bounds__(T) void k_quant_tok_grp(const float* x, int xstride, int K, int gs, int8_t* xq,
-                                                     float* xs, float gq) {
+                                                     float* xs) {
     const int g = blockIdx.x, tok = blockIdx.y, t = threadIdx.x, ng = K / gs;
     __shared__ float red[T / 64];
     const float* row = x + (size_t)tok * xstride + (size_t)g * gs;
     int8_t* out = xq + (size_t)tok * K + (size_t)g * gs;
     if constexpr (NV > 0) {
-        quant_group<T, NV>([&](int k) { return *(const float4*)(row + k); }, gs, gq, out, xs + (size_t)tok * ng + g, red);
+        quant_group<T, NV>([&](int k) { return *(const float4*)(row + k); }, gs, 1.0f, out, xs + (size_t)tok * ng + g, red);
     } else {
         float mx = 0.0f;
         for (int k = 4 * t; k < gs; k += 4 * T) {
@@ -942,7 +942,7 @@ __global__ __launch_bounds__(T) void k_quant_tok_grp(const float* x, int xstride
         float m = red[0];
 #pragma unroll
         for (int w = 1; w < T / 64; ++w) m = fmaxf(m, red[w]);
-        const float sc = m * gq * (1.0f / 127.0f), qi = (sc > 0.0f) ? gq / sc : 0.0f;   // gq = 1/in_scale
+        const float sc = m * (1.0f / 127.0f), qi = (sc > 0.0f) ? 1.0f / sc : 0.0f;
         if (t == 0) xs[(size_t)tok * ng + g] = sc;
         for (int k = 4 * t; k < gs; k += 4 * T) {
             const float4 v = *(const float4*)(row + k);
@@ -950,9 +950,9 @@ __global__ __launch_bounds__(T) void k_quant_tok_grp(const float* x, int xstride
         }
     }
 }
-static int run_quant_tok_grp(const float* x, int xstride, int M, int K, int gs, int8_t* xq, float* xs, float gq, hipStream_t s) {
+static int run_quant_tok_grp(const float* x, int xstride, int M, int K, int gs, int8_t* xq, float* xs, hipStream_t s) {
     const dim3 grid((unsigned)(K / gs), (unsigned)M);
-#define Q27X_QT(T, NV) hipLaunchKernelGGL((k_quant_tok_grp<T, NV>), grid, dim3(T), 0, s, x, xstride, K, gs, xq, xs, gq)
+#define Q27X_QT(T, NV) hipLaunchKernelGGL((k_quant_tok_grp<T, NV>), grid, dim3(T), 0, s, x, xstride, K, gs, xq, xs)
     if (gs <= 1024) Q27X_QT(256, 1);
     else if (gs <= 2048) Q27X_QT(256, 2);
     else if (gs <= 4096) Q27X_QT(256, 4);
@@ -990,7 +990,7 @@ extern "C" int q27x_quant_tok_groups(const float* x, int xstride, int M, int K, 
         set_error("q27x_quant_tok_groups: bad arguments (M %d, K %d, gs %d, xstride %d)", M, K, gs, xstride);
         return Q27X_E_ARG;
     }
-    return run_quant_tok_grp(x, xstride, M, K, gs, xq, xs, 1.0f, (hipStream_t)s);
+    return run_quant_tok_grp(x, xstride, M, K, gs, xq, xs, (hipStream_t)s);
 }
 
 extern "C" int q27x_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, float alpha, const int8_t* x,
@@ -1190,16 +1190,6 @@ int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, floa
     }
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
-}
-// the per-(token, group) quantizer with g = 1/in_scale (s = mx g / 127, qi = g / s)
-int launch_quant_tok_grp(const float* x, int xstride, int M, int K, int gs, float in_scale, int8_t* xq, float* xs,
-                         hipStream_t s) {
-    if (!x || !xq || !xs || M < 1 || K < 4 || gs < 4 || (gs & 3) || (K % gs) || xstride < K || (xstride & 3) ||
-        ((uintptr_t)x & 15) || !(in_scale > 0.0f)) {
-        set_error("quant tok groups: bad arguments (M %d, K %d, gs %d)", M, K, gs);
-        return Q27X_E_ARG;
-    }
-    return run_quant_tok_grp(x, xstride, M, K, gs, xq, xs, 1.0f / in_scale, s);
 }
 
 }  // namespace q27x

@@ -33,7 +33,6 @@ struct NormArgs {
     const int* stop;
     const int* row_sel;                           // optional: process only row *row_sel (into row 0)
     unsigned long long* stamp;                    // optional: block 0 stores the wall clock at its start
-    float* yf; int yfstride;                      // optional: the values xq would quantize, as fp32
 };
 // ---------------------------------------------------------------- projection
 enum ProjEpi { EPI_STORE = 0, EPI_SWIGLU = 2, EPI_CONV = 3 };
@@ -114,6 +113,7 @@ int launch_argmax_rows(const float* logits, int n, int ld, int nr, int32_t* idx,
                        float* pval, uint32_t* pidx, hipStream_t s);
 
 int launch_norm(const NormArgs& a, int nr, hipStream_t s);
+int launch_norm_grp(const NormArgs& a, int nr, int gs, hipStream_t s);
 int launch_quant_rows(const uint16_t* x, int xstride, int8_t* xq, int qstride, float* xs,
                       int sstride, int n, float in_scale, int nrows, hipStream_t s);
 int launch_swiglu(const float* g, const float* u, int stride, int8_t* xq, float* xs, int n,
@@ -180,8 +180,6 @@ int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, floa
 
 // ---------------------------------------------------------------- prefill element kernels (k_prefill.hip)
 int launch_pf_quant_bf16(const uint16_t* x, int ld, int M, int K, int gs, float in_scale, int8_t* xq, float* xs,
-                         hipStream_t s);
-int launch_quant_tok_grp(const float* x, int xstride, int M, int K, int gs, float in_scale, int8_t* xq, float* xs,
                          hipStream_t s);
 int launch_pf_conv(const uint16_t* buf, int ld, int C, int nconv, const uint16_t* conv_w, uint16_t* rec, int npend,
                    uint16_t* out, int ldo, hipStream_t s);

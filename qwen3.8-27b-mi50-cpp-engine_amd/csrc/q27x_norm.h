@@ -13,8 +13,9 @@
 namespace q27x {
 
 // Rows [r0, r0 + nrows) of `a` (source row index rs = row_sel ? *row_sel : r), RB rows per pass.
-// NCH = n / 1024. wsum: __shared__ float[RB][4]. Every thread of the 256-thread block calls it.
-template <int NCH, int RB>
+// NCH = n / 1024. wsum: __shared__ float[RB][4]. Every thread of the 256-thread block calls it. GM: xq/xs hold codes
+// per 16 columns (0), per row (1) or per 1024 columns (2).
+template <int NCH, int RB, int GM = 0>
 __device__ __forceinline__ void norm_rows(const NormArgs& a, int r0, int nrows, float (*wsum)[4]) {
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     constexpr int n = NCH * 1024;
@@ -102,11 +103,10 @@ __device__ __forceinline__ void norm_rows(const NormArgs& a, int r0, int nrows, 
                 if (a.y)
                     *(uint2*)(a.y + (size_t)r * a.ystride + k) = make_uint2((uint32_t)yb[0] | ((uint32_t)yb[1] << 16),
                                                                            (uint32_t)yb[2] | ((uint32_t)yb[3] << 16));
-                if (a.yf)
-                    *(float4*)(a.yf + (size_t)r * a.yfstride + k) =
-                        a.quant_bf16 ? make_float4(bf2f(yb[0]), bf2f(yb[1]), bf2f(yb[2]), bf2f(yb[3]))
-                                     : make_float4(nm[0], nm[1], nm[2], nm[3]);
-                if (a.xq) {
+                if constexpr (GM != 0) {           // codes below, once the row's maximum is known
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) xv[j][i][e] = a.quant_bf16 ? bf2f(yb[e]) : nm[e];
+                } else if (a.xq) {
                     float q[4], mx = 0.0f;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { q[e] = a.quant_bf16 ? bf2f(yb[e]) : nm[e]; mx = fmaxf(mx, fabsf(q[e])); }
@@ -119,6 +119,42 @@ __device__ __forceinline__ void norm_rows(const NormArgs& a, int r0, int nrows, 
                     *(uint32_t*)(a.xq + (size_t)r * n + k) = pk;
                     if ((t & 3) == 0) a.xs[(size_t)r * (n >> 4) + (k >> 4)] = s;
                 }
+            }
+        }
+        if constexpr (GM != 0) {
+            // codes per (row, group) from the registers: group = the row, or each 1024 columns (k_quant_tok_grp's scale
+            // and codes)
+            static_assert(RB == 1, "one row per pass");
+            __shared__ float red[NCH][4];
+            constexpr int NG = GM == 1 ? 1 : NCH;
+            const int r = r0 + rb;
+            float mx[NG];
+#pragma unroll
+            for (int i = 0; i < NG; ++i) mx[i] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NCH; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mx[i % NG] = fmaxf(mx[i % NG], fabsf(xv[0][i][e]));
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                mx[i] = max_xor(mx[i], 64);
+                if (lane == 0) red[i][wv] = mx[i];
+            }
+            __syncthreads();
+            float qi[NG];
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                const float m = fmaxf(fmaxf(fmaxf(red[i][0], red[i][1]), red[i][2]), red[i][3]);
+                const float s = m * g * (1.0f / 127.0f);
+                qi[i] = (s > 0.0f) ? (g / s) : 0.0f;
+                if (t == 0) a.xs[(size_t)r * NG + i] = s;
+            }
+#pragma unroll
+            for (int i = 0; i < NCH; ++i) {
+                const float* v = xv[0][i];
+                const float q = qi[i % NG];
+                *(uint32_t*)(a.xq + (size_t)r * n + i * 1024 + 4 * t) =
+                    pack4(qcode(v[0], q), qcode(v[1], q), qcode(v[2], q), qcode(v[3], q));
             }
         }
         __syncthreads();   // wsum reused by the next pass
