@@ -135,7 +135,8 @@ int launch_pf_conv(const uint16_t* buf, int ld, int C, int nconv, const uint16_t
 // against every staged row, so a staged value is read and widened once for two rows. Bound by VALU
 // issue (3 instructions per two products; one row per wave with both operands widened at the
 // product took 6, on half the CUs): 1024 rows x 96 x 5120 92 -> 76 us
-// beside another chunk's scan, which holds 96 CUs.
+// beside another chunk's scan, which holds 96 CUs. The logits of a block's rows wait in the lanes and become decay and
+// beta at once (row by row, by two lanes each time: 1500 rows 111 us beside other kernels, so 99).
 constexpr int kAbTok = 8;            // rows per block
 constexpr int kAbWaves = 8;          // waves per block, two weight rows each
 constexpr int kAbChunks = 10;        // weight chunks per lane at most (K <= 5120)
@@ -145,9 +146,9 @@ template <int KC>
 __global__ __launch_bounds__(64 * kAbWaves) void k_pf_ab(const uint16_t* __restrict__ in_a, const uint16_t* __restrict__ in_b,
                                                 const uint16_t* __restrict__ A_log,
                                                 const uint16_t* __restrict__ dt_bias, const uint16_t* __restrict__ y,
-                                                int ystride, int K, int vh, int C, float* __restrict__ out) {
-    extern __shared__ uint4 sy[];                 // [kAbTok][K / 8] chunks
-    const int t0 = blockIdx.x * kAbTok, nt = (C - t0 < kAbTok) ? C - t0 : kAbTok;
+                                                int ystride, int K, int vh, int C, int tb, float* __restrict__ out) {
+    extern __shared__ uint4 sy[];                 // [tb][K / 8] chunks
+    const int t0 = blockIdx.x * tb, nt = (C - t0 < tb) ? C - t0 : tb;      // tb <= kAbTok rows
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nch = K >> 3;
     for (int i = threadIdx.x; i < nt * nch; i += 64 * kAbWaves) {
@@ -178,10 +179,8 @@ __global__ __launch_bounds__(64 * kAbWaves) void k_pf_ab(const uint16_t* __restr
     }
     __syncthreads();
     if (j0 >= 2 * vh) return;
-    // lanes 0 and 1 turn the two rows' logits into decay = exp(-exp(A_log) softplus(a + dt)) or beta = sigmoid(b)
-    const int j = j0 + (lane & 1), which = j >= vh, head = j - which * vh;
-    const float Aexp = which ? 0.0f : qexp(bf2f(A_log[head]));
-    const float dtb = which ? 0.0f : bf2f(dt_bias[head]);
+    // lanes 2 n and 2 n + 1 keep row n's two logits
+    float v = 0.0f;
     for (int n = 0; n < nt; ++n) {
         const uint4* yr = sy + (size_t)n * nch;
         float acc[2] = {0.0f, 0.0f};
@@ -201,11 +200,15 @@ __global__ __launch_bounds__(64 * kAbWaves) void k_pf_ab(const uint16_t* __restr
             }
         }
         const float a0 = bcast0(tree64(acc[0])), a1 = bcast0(tree64(acc[1]));
-        const float v = bfr((lane & 1) ? a1 : a0);
-        if (lane < 2) {
-            const float r = which ? qsigmoid(v) : qexp(-(Aexp * qsoftplus(v + dtb)));
-            out[((size_t)which * C + t0 + n) * vh + head] = r;
-        }
+        v = (lane >> 1) == n ? ((lane & 1) ? a1 : a0) : v;
+    }
+    if (lane < 2 * nt) {        // decay = exp(-exp(A_log) softplus(a + dt)) or beta = sigmoid(b), all rows at once
+        const int j = j0 + (lane & 1), which = j >= vh, head = j - which * vh;
+        v = bfr(v);
+        float r;
+        if (which) r = qsigmoid(v);
+        else r = qexp(-(qexp(bf2f(A_log[head])) * qsoftplus(v + bf2f(dt_bias[head]))));
+        out[((size_t)which * C + t0 + (lane >> 1)) * vh + head] = r;
     }
 }
 int launch_pf_ab(const uint16_t* in_a, const uint16_t* in_b, const uint16_t* A_log, const uint16_t* dt_bias,
@@ -215,7 +218,6 @@ int launch_pf_ab(const uint16_t* in_a, const uint16_t* in_b, const uint16_t* A_l
         set_error("prefill a/b: bad arguments");
         return Q27X_E_ARG;
     }
-    const size_t lds = (size_t)kAbTok * (K / 8) * 16;
     static bool lds_set = false;
     const int mx = kAbTok * 64 * kAbChunks * 16;
     if (!lds_set) {
@@ -226,11 +228,17 @@ int launch_pf_ab(const uint16_t* in_a, const uint16_t* in_b, const uint16_t* A_l
         lds_set = true;
     }
     const int kc = (K / 8 + 63) / 64;
-    const dim3 grid((unsigned)((C + kAbTok - 1) / kAbTok), (unsigned)((vh + kAbWaves - 1) / kAbWaves)), blk(64 * kAbWaves);
-    if (kc <= 2) hipLaunchKernelGGL(k_pf_ab<2>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else if (kc <= 4) hipLaunchKernelGGL(k_pf_ab<4>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else if (kc <= 8) hipLaunchKernelGGL(k_pf_ab<8>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
-    else hipLaunchKernelGGL(k_pf_ab<10>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, out);
+    // kAbTok rows per block once that fills the chip, fewer for short chunks (a block's time is its rows one after the
+    // other): 40 rows x 96 x 5120 in 30 blocks of 8 rows 19.7 us, in 240 blocks of one 7.7
+    const int gy = (vh + kAbWaves - 1) / kAbWaves;
+    int tb = (int)(((long long)C * gy + 255) / 256);
+    tb = tb < 1 ? 1 : tb > kAbTok ? kAbTok : tb;
+    const size_t lds = (size_t)tb * (K / 8) * 16;
+    const dim3 grid((unsigned)((C + tb - 1) / tb), (unsigned)gy), blk(64 * kAbWaves);
+    if (kc <= 2) hipLaunchKernelGGL(k_pf_ab<2>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, tb, out);
+    else if (kc <= 4) hipLaunchKernelGGL(k_pf_ab<4>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, tb, out);
+    else if (kc <= 8) hipLaunchKernelGGL(k_pf_ab<8>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, tb, out);
+    else hipLaunchKernelGGL(k_pf_ab<10>, grid, blk, lds, s, in_a, in_b, A_log, dt_bias, y, ystride, K, vh, C, tb, out);
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
 }

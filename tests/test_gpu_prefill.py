@@ -85,6 +85,12 @@ def test_tiny_prefill_scan_row_edges_match_oracle(gpu, O, n):
     run_case(gpu, O, gpu.tiny_config(spec_k=2), n, 1)
 
 
+@pytest.mark.parametrize("n", [101, 235])
+def test_full_width_prefill_ab_row_splits_match_oracle(gpu, O, n):
+    """The a/b kernel's rows per block (3 at 101 rows, 6 at 235) with a last block of 2 and of 1."""
+    run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=512), n, 1)
+
+
 def test_tiny_wide_group_swiglu_prefill_matches_oracle(gpu, O):
     """inter 5120 with whole-K groups: the down projection's input is quantized per (token, 5120)
     by the wide-group SwiGLU kernel (values held in registers: 1280 quads on 1024 threads, the
