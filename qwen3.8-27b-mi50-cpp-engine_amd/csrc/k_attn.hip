@@ -181,20 +181,6 @@ constexpr int kSplitBlocks = 256;
 // here (once per block) instead of read back, and the split that holds
 // the step's new positions computes their K and V, writes them to the cache and puts the
 // dequantized values straight into its tile.
-// Row tiles (a.zrows > 0, prefill): block z of grid.z works on rows z zrows .. of the query rows,
-// at their positions, with its own work region, exactly as a launch of those rows alone would.
-template <int HD = kHD>
-__device__ __forceinline__ void tile_rows(AttnArgs& a, int nr, int& pos0, int& nact) {
-    const int z = blockIdx.z;
-    const int r0 = z * a.zrows;
-    pos0 += r0;
-    nact = (a.ztotal - r0 < a.zrows) ? a.ztotal - r0 : a.zrows;
-    a.qh += (size_t)r0 * a.nq * HD;
-    a.qkv += (size_t)r0 * a.qkv_stride;
-    a.work += (size_t)z * nr * a.nq * a.max_splits * (size_t)(HD + 2);   // attn_work_floats of the tile
-    a.out += (size_t)r0 * a.nq * HD;
-    if (a.xq) { a.xq += (size_t)r0 * a.nq * HD; a.xs += (size_t)r0 * a.nq * HD / 16; }
-}
 template <int NQW, int QPT, bool PREP>
 __global__ __launch_bounds__(kAttnThreads) void k_attn_split(AttnArgs a, int nr) {
     warm_args(a);
@@ -204,7 +190,6 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn_split(AttnArgs a, int nr)
     const int gsq = __builtin_ctz(G);               // G is a power of two: query i = (row i >> gsq, head i & (G - 1))
     int nact = a.nact_ptr ? ld_uniform(a.nact_ptr) : nr;
     int pos0 = a.pos0_ptr ? ld_uniform(a.pos0_ptr) : a.pos0_imm;
-    if (!PREP && a.zrows) tile_rows(a, nr, pos0, nact);
     const int Lmax = pos0 + nact;
     const int nqr = nact * G;                       // query vectors of this kv head
     const int kvrows = a.nkv * kHD;
@@ -591,7 +576,7 @@ __global__ __launch_bounds__(HD) void k_attn_combine(AttnArgs a, int nr) {
 
 // ---------------------------------------------------------------- general geometry
 // Heads of HD = 256 dims (the reference trunk's 24q / 4kv x 256, include/q27.h:25-35) or GQA groups
-// that are not a power of two. Queries come from qh (the prep runs as its own launch before), K and
+// that are not a power of two, and the row tiles of a prefill. Queries come from qh (the prep runs as its own launch before), K and
 // V from the cache. The splits, and the order of every sum, are those of the kernels above and of
 // the oracle: score = ((c0 + c1) + c2) + c3 with c_j the fmaf chain over dims [j HD/4, (j+1) HD/4),
 // on K values code x scale; the split softmax m = max, p = 2^(x - m), l = the 64-lane shfl_down
@@ -625,6 +610,20 @@ constexpr int kSpG = kSplit + 4;                 // score row stride (floats)
 template <int HD>
 __host__ __device__ constexpr size_t split_g_lds(int qt, int nsc) {
     return (size_t)2 * kSplit * HD + (size_t)2 * kSplit * nsc * 4 + (size_t)qt * 16 * kSpG * 4;
+}
+// Row tiles (a.zrows > 0, prefill): block z of grid.z works on rows z zrows .. of the query rows,
+// at their positions, with its own work region, exactly as a launch of those rows alone would.
+template <int HD>
+__device__ __forceinline__ void tile_rows(AttnArgs& a, int nr, int& pos0, int& nact) {
+    const int z = blockIdx.z;
+    const int r0 = z * a.zrows;
+    pos0 += r0;
+    nact = (a.ztotal - r0 < a.zrows) ? a.ztotal - r0 : a.zrows;
+    a.qh += (size_t)r0 * a.nq * HD;
+    a.qkv += (size_t)r0 * a.qkv_stride;
+    a.work += (size_t)z * nr * a.nq * a.max_splits * (size_t)(HD + 2);   // attn_work_floats of the tile
+    a.out += (size_t)r0 * a.nq * HD;
+    if (a.xq) { a.xq += (size_t)r0 * a.nq * HD; a.xs += (size_t)r0 * a.nq * HD / 16; }
 }
 template <int HD, int QT>
 __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int nr) {
@@ -903,10 +902,14 @@ __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int n
     }
 }
 
-// The 128-wide kernels above need a power-of-two GQA group; the general kernel takes the rest.
+// The 128-wide kernels above need a power-of-two GQA group; the general kernel takes the rest, and every
+// prefill's row tiles: up to 64 query vectors and separate prep anyway, and its two blocks per CU cover each
+// other's softmax (32q / 8kv x 128, 64 layers: ingest of 4096 tokens 228 -> 209 ms, of
+// 16320 1.44 -> 1.28 s, of 1024 and less the same). A verify step keeps the kernels above,
+// which save the prep's launch.
 static bool attn_general(const AttnArgs& a) {
     const int G = a.nq / a.nkv;
-    return a.hd != kHD || (G & (G - 1));
+    return a.hd != kHD || (G & (G - 1)) || a.zrows;
 }
 
 static int attn_check(const AttnArgs& a, int nr) {
@@ -987,7 +990,7 @@ static int launch_split(const AttnArgs& a, int nr, hipStream_t s) {
     }
     // at most kSplitBlocks blocks (about one per CU); a block takes splits blockIdx.x + i gridDim.x
     const int bx = a.max_splits < kSplitBlocks / a.nkv ? a.max_splits : (kSplitBlocks / a.nkv > 0 ? kSplitBlocks / a.nkv : 1);
-    const dim3 grid(bx, a.nkv, a.zrows ? (unsigned)((a.ztotal + a.zrows - 1) / a.zrows) : 1u);
+    const dim3 grid(bx, a.nkv);
     if (nqr <= 8) hipLaunchKernelGGL((k_attn_split<1, 1, PREP>), grid, dim3(kAttnThreads), lds, s, a, nr);
     else if (nqr <= 16) hipLaunchKernelGGL((k_attn_split<2, 1, PREP>), grid, dim3(kAttnThreads), lds, s, a, nr);
     else if (nqr <= 24) hipLaunchKernelGGL((k_attn_split<3, 2, PREP>), grid, dim3(kAttnThreads), lds, s, a, nr);
