@@ -91,6 +91,13 @@ def test_full_width_prefill_ab_row_splits_match_oracle(gpu, O, n):
     run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=512), n, 1)
 
 
+@pytest.mark.parametrize("nq,nkv,n", [(4, 4, 67), (4, 2, 130), (8, 1, 67)])
+def test_tiny_prefill_attention_groups_match_oracle(gpu, O, nq, nkv, n):
+    """128-wide heads in GQA groups of 1, 2 and 8 (one, two and four query tiles per block, row tiles of 16 and 8
+    rows with a remainder, splits that a row tile straddles)."""
+    run_case(gpu, O, gpu.tiny_config(spec_k=2, n_q=nq, n_kv=nkv), n, 2)
+
+
 def test_tiny_wide_group_swiglu_prefill_matches_oracle(gpu, O):
     """inter 5120 with whole-K groups: the down projection's input is quantized per (token, 5120)
     by the wide-group SwiGLU kernel (values held in registers: 1280 quads on 1024 threads, the
