@@ -147,6 +147,10 @@ int q27x_quant_tok_groups(const float* x, int xstride, int M, int K, int gs, int
 int q27x_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, float alpha,
                   const int8_t* x, const float* sx, int M, float* y, int ldy, const float* res,
                   int ldr, float rs, q27x_stream_t s);
+/* The kernel form q27x_gemm_i8g launches for a shape (ldy = N, no residual), by the same rule and without a device: its
+ * index in the launcher's list (what the environment's Q27X_GEMM_FORM names; one list for gs == K, one for several
+ * groups), and in *bm, *bn (may be NULL) the tokens and weight rows of a block. Negative: the shape is refused. */
+int q27x_gemm_i8g_form(int M, int N, int K, int gs, int* bm, int* bn);
 
 /* R9 / lm_head bf16 GEMV of nr rows (replaces q27_bf16_gemv2_tile, include/q27_nr.h:75-76):
  *   y[n][r] = sum_k bf16(W[r][k]) * bf16(x[n][k]) in fp32; out_bf16 selects bf16 / fp32 out.

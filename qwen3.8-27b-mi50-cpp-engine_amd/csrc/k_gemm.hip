@@ -17,14 +17,15 @@
 // The int32 group sums do not depend on the order of their terms, so the MFMA tiling cannot
 // change them; the fp32 part runs per output in the reference's group order.
 //
-// GEMM tiling: a launch takes the cheapest of a list of forms (launch_gemm_i8g): k_gemm_i8g_ring (64 to 256 tokens
+// GEMM tiling: a launch takes the cheapest of a list of forms (pick_form): k_gemm_i8g_ring (64 to 256 tokens
 // x 64 to 256 weight rows per block, 128-byte K stages in an LDS ring), k_gemm_i8g_sk (few tokens: small tiles whose
-// waves split K), k_gemm_i8g_w4 (256 x 256 tiles, one group over K) and k_gemm_i8g_rs (256 x 128, many groups). At
+// waves split K), k_gemm_i8g_w4 (256 x 256 tiles, one group over K) and k_gemm_i8g_rs (256 x 128, several groups). At
 // the end of each group the int32 tiles are folded into fp32 accumulators with the group's scales and restarted
 // from zero. The general form for the other shapes, k_gemm_i8g: a 256-thread block computes a 128-token x 128-row
 // tile; wave w owns the 64 x 64 quarter (w / 2, w % 2) as 2 x 2 v_mfma_i32_32x32x32_i8 tiles, and two blocks share a
 // CU. K advances 64 bytes per stage through a ring of 4 LDS stages (3 when the scales of 17+ groups take the room)
 // filled by LDS DMA ahead of the multiply.
+#include <math.h>
 #include <stdlib.h>
 #include <mutex>
 #include <type_traits>
@@ -1075,73 +1076,128 @@ static int run_gemm_rs(const GemmArgs& a, hipStream_t s) {
     return Q27X_OK;
 }
 
-// The kernel forms and what a launch of each costs. A CU takes n = ceil(blocks / CUs) blocks, occ at a time; a block
-// runs K / 128 (/ ks) stages, t[r - 1] us per stage with r blocks on the CU; all blocks together read
-// (bm + bn) K bytes each at bw TB/s, and the weights come from HBM at 4.9 TB/s:
-//   us = a + max(stages (floor(n / occ) t[occ - 1] + t[n % occ - 1]), blocks (bm + bn) K / bw, N K / 4.9)
-// The constants are fits of measured launches (M = 1 .. 4096 at the model's nine widths, 216 shapes; per group of
-// 1024 columns 65 shapes). Over these the form taken is 3% off the fastest one on average. Before (128 x 128 tiles
-// of 64-byte stages below 512 tokens; from there 256 x 128 or 256 x 256) and now, us: M = 1, 5120 x 17408: 86 / 19;
-// M = 77: 102 / 33 (1024-column groups 125 / 45); M = 203, 5120 x 17408: 101 / 62, 34816 x 5120: 105 / 87;
-// M = 512: 129 / 82, 153 / 132; M = 1024, 5120 x 17408: 147 / 118; the 256 x 256 tiles stay for 1024 x 34816 up.
-enum { F_RING, F_SK, F_W4, F_RS };
+// The kernel forms and what a launch of each costs. A CU takes n = ceil(blocks / CUs) blocks, occ at a time; r blocks on
+// a CU run their K / 128 (/ ks) stages and (with several groups) K / gs folds in T(r) = e + h r + stages t[r - 1] + folds
+// g r us; all blocks together read (bm + bn) K bytes each at bw TB/s (100: no such bound seen), and the weights and
+// outputs move at hb TB/s:
+//   us = a + |(floor(n / occ) T(occ) + T(n % occ), blocks (bm + bn) K / bw, (N K + 4 M N) / hb)|
+// (the root of the squares: the three overlap, but not fully where they are alike). The constants are fits of measured
+// launches, on weights that a cache holds and on weights that none holds: 2941 shapes, M 1 to 4096, N 128 to 62080, K 128
+// to 19200, one group and groups of 128 columns and more. The form taken is 0.5% (several groups) and 1.2% (one) off the
+// fastest one on average. A cost without e, h and g, with constants from long K and groups of 1024 columns, was 5 to 6%
+// off: it took split-K tiles of many short blocks, or too many folds, where larger tiles are up to 2.7 times as fast: us
+// for 33 x 36864 x 512 27, now 10; 512 x 4096 x 256 in groups of 128 25 / 9; 384 x 14336 x 5120 in groups of 256 93 / 70.
+// Against 128 x 128 tiles of 64-byte stages below 512 tokens and 256 x 128 or 256 x 256 ones from there: M = 1, 5120 x
+// 17408: 86 / 20; M = 77: 102 / 33 (1024-column groups 125 / 45); M = 203, 34816 x 5120: 105 / 87; M = 512: 153 / 132;
+// M = 1024, 5120 x 17408: 147 / 118.
+enum { F_RING, F_SK, F_W4, F_RS, F_GEN };
 struct GemmForm {
     int kind, bm, bn, ks, occ;
-    float a, t[3], bw;
+    float a, e, h, g, t[3], bw, hb;
     int (*run)(const GemmArgs&, hipStream_t);
 };
 static int run_w4(const GemmArgs& a, hipStream_t s) { return a.out_bf16 ? run_gemm_w4<true>(a, s) : run_gemm_w4<false>(a, s); }
 static int run_rs(const GemmArgs& a, hipStream_t s) { return a.out_bf16 ? run_gemm_rs<true>(a, s) : run_gemm_rs<false>(a, s); }
-// one group over K
+// 64-byte stages: token tiles of 256 (8 waves, one block per CU, a 5-stage ring) or 128 (4 waves, two blocks per CU, a
+// 4-stage ring, or 3 when 17+ groups' scales take the room)
+static int run_gen256(const GemmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)(a.N / kGN) * (unsigned)((a.M + 255) / 256));
+    hipLaunchKernelGGL((k_gemm_i8g<256, 5>), grid, dim3(512), (size_t)(256 + kGN) * a.ng * sizeof(float), s, a);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+static int run_gen128(const GemmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)(a.N / kGN) * (unsigned)((a.M + 127) / 128));
+    const size_t scl = (size_t)(128 + kGN) * a.ng * sizeof(float);
+    if (64 * 1024 + scl <= 80 * 1024) hipLaunchKernelGGL((k_gemm_i8g<128, 4>), grid, dim3(256), scl, s, a);
+    else hipLaunchKernelGGL((k_gemm_i8g<128, 3>), grid, dim3(256), scl, s, a);
+    Q27X_HIP(hipGetLastError());
+    return Q27X_OK;
+}
+// one group over K (the last three: shapes that the others do not take)
 static const GemmForm kFormsK[] = {
-    {F_SK, 16, 32, 4, 2, 3.57f, {0.316f, 0.653f}, 13.7f, run_gemm_sk<2, 1, 4, 3>},
-    {F_SK, 32, 32, 4, 2, 3.75f, {0.412f, 0.821f}, 16.0f, run_gemm_sk<2, 2, 4, 2>},
-    {F_SK, 32, 32, 2, 3, 4.19f, {0.337f, 0.450f, 0.505f}, 15.6f, run_gemm_sk<2, 2, 2, 2>},
-    {F_SK, 32, 64, 4, 1, 4.16f, {0.738f}, 13.7f, run_gemm_sk<4, 2, 4, 2>},
-    {F_SK, 64, 64, 4, 1, 6.34f, {0.983f}, 15.4f, run_gemm_sk<4, 4, 4, 2>},
-    {F_RING, 64, 64, 1, 3, 5.41f, {0.239f, 0.456f, 0.605f}, 15.2f, run_gemm_ring<1, 1, 2, 3, false>},
-    {F_RING, 64, 128, 1, 2, 5.93f, {0.309f, 0.793f}, 15.1f, run_gemm_ring<1, 2, 2, 3, false>},
-    {F_RING, 64, 256, 1, 1, 5.70f, {0.755f}, 13.0f, run_gemm_ring<1, 4, 1, 3, false>},
-    {F_RING, 128, 128, 1, 1, 4.40f, {0.534f}, 11.8f, run_gemm_ring<2, 2, 2, 3, false>},
-    {F_RING, 128, 256, 1, 1, 4.39f, {1.013f}, 10.7f, run_gemm_ring<2, 4, 1, 3, false>},
-    {F_RING, 256, 128, 1, 1, 3.87f, {0.935f}, 10.9f, run_gemm_ring<4, 2, 1, 3, false>},
-    {F_W4, 256, 256, 1, 1, 1.40f, {1.770f}, 7.9f, run_w4},
+    {F_SK, 16, 32, 4, 2, 2.10f, 1.50f, 0.09f, 0.00f, {0.355f, 0.641f}, 39.1f, 5.11f, run_gemm_sk<2, 1, 4, 3>},
+    {F_SK, 32, 32, 4, 2, 1.69f, 1.49f, 0.67f, 0.00f, {0.420f, 0.793f}, 26.2f, 5.79f, run_gemm_sk<2, 2, 4, 2>},
+    {F_SK, 32, 64, 4, 1, 1.25f, 4.26f, 0.00f, 0.00f, {0.694f}, 47.8f, 5.29f, run_gemm_sk<4, 2, 4, 2>},
+    {F_RING, 64, 64, 1, 3, 2.10f, 1.38f, 0.95f, 0.00f, {0.300f, 0.460f, 0.605f}, 34.0f, 5.27f, run_gemm_ring<1, 1, 2, 3, false>},
+    {F_RING, 64, 128, 1, 2, 1.83f, 0.80f, 2.16f, 0.00f, {0.298f, 0.566f}, 25.6f, 5.11f, run_gemm_ring<1, 2, 2, 3, false>},
+    {F_RING, 64, 256, 1, 1, 0.11f, 5.32f, 0.00f, 0.00f, {0.623f}, 28.0f, 3.88f, run_gemm_ring<1, 4, 1, 3, false>},
+    {F_RING, 128, 128, 1, 1, 0.00f, 4.58f, 0.00f, 0.00f, {0.399f}, 17.6f, 5.03f, run_gemm_ring<2, 2, 2, 3, false>},
+    {F_RING, 128, 256, 1, 1, 0.11f, 5.74f, 0.00f, 0.00f, {0.805f}, 21.9f, 4.39f, run_gemm_ring<2, 4, 1, 3, false>},
+    {F_RING, 256, 128, 1, 1, 0.19f, 6.21f, 0.00f, 0.00f, {0.689f}, 17.3f, 5.19f, run_gemm_ring<4, 2, 1, 3, false>},
+    {F_W4, 256, 256, 1, 1, 0.25f, 7.61f, 0.00f, 0.00f, {1.300f}, 12.6f, 5.21f, run_w4},
+    {F_GEN, 128, 128, 1, 2, 0.0f, 0.0f, 0.0f, 0.0f, {1.0f, 1.0f}, 100.0f, 5.0f, run_gen128},
+    {F_GEN, 256, 128, 1, 1, 0.0f, 0.0f, 0.0f, 0.0f, {1.0f}, 100.0f, 5.0f, run_gen256},
+    {F_RS, 256, 128, 1, 1, 0.0f, 0.0f, 0.0f, 0.0f, {1.0f}, 100.0f, 5.0f, run_rs},
 };
 // several groups
 static const GemmForm kFormsG[] = {
-    {F_SK, 16, 32, 4, 2, 3.50f, {0.535f, 1.343f}, 20.0f, run_gemm_sk<2, 1, 4, 3>},
-    {F_SK, 32, 32, 8, 1, 3.23f, {1.383f}, 11.4f, run_gemm_sk<2, 2, 8, 2>},
-    {F_SK, 32, 64, 4, 1, 3.55f, {1.343f}, 20.0f, run_gemm_sk<4, 2, 4, 2>},
-    {F_RING, 64, 64, 1, 2, 4.71f, {0.701f, 0.758f}, 14.0f, run_gemm_ring<1, 1, 1, 4, true>},
-    {F_RING, 64, 128, 1, 2, 5.04f, {0.593f, 1.028f}, 12.7f, run_gemm_ring<1, 2, 1, 3, true>},
-    {F_RING, 64, 256, 1, 1, 4.91f, {0.795f}, 11.6f, run_gemm_ring<1, 4, 1, 3, true>},
-    {F_RING, 128, 128, 1, 1, 4.93f, {0.677f}, 10.0f, run_gemm_ring<2, 2, 1, 4, true>},
-    {F_RING, 128, 256, 1, 1, 4.05f, {1.095f}, 9.0f, run_gemm_ring<2, 4, 1, 3, true>},
-    {F_RING, 256, 128, 1, 1, 4.77f, {0.964f}, 9.2f, run_gemm_ring<4, 2, 1, 3, true>},
-    {F_RS, 256, 128, 1, 1, 6.23f, {0.961f}, 8.0f, run_rs},
+    {F_SK, 16, 32, 4, 2, 0.95f, 1.89f, 0.41f, 0.24f, {0.352f, 0.829f}, 100.0f, 4.80f, run_gemm_sk<2, 1, 4, 3>},
+    {F_SK, 32, 32, 8, 1, 1.10f, 2.01f, 0.00f, 0.27f, {0.830f}, 18.9f, 4.95f, run_gemm_sk<2, 2, 8, 2>},
+    {F_SK, 32, 64, 4, 1, 1.32f, 3.24f, 0.00f, 0.69f, {0.715f}, 100.0f, 4.71f, run_gemm_sk<4, 2, 4, 2>},
+    {F_RING, 64, 128, 1, 2, 2.91f, 1.73f, 0.09f, 1.17f, {0.438f, 0.934f}, 27.1f, 5.46f, run_gemm_ring<1, 2, 1, 3, true>},
+    {F_RING, 64, 256, 1, 1, 0.59f, 3.83f, 0.00f, 1.38f, {0.565f}, 34.5f, 5.22f, run_gemm_ring<1, 4, 1, 3, true>},
+    {F_RING, 128, 128, 1, 1, 0.32f, 4.61f, 0.00f, 1.22f, {0.476f}, 25.0f, 5.55f, run_gemm_ring<2, 2, 1, 4, true>},
+    {F_RING, 128, 256, 1, 1, 0.06f, 4.98f, 0.00f, 0.92f, {0.729f}, 17.5f, 4.94f, run_gemm_ring<2, 4, 1, 3, true>},
+    {F_RING, 256, 128, 1, 1, 0.15f, 4.97f, 0.00f, 0.98f, {0.668f}, 16.2f, 6.54f, run_gemm_ring<4, 2, 1, 3, true>},
+    {F_RS, 256, 128, 1, 1, 2.08f, 3.24f, 0.00f, 1.05f, {0.810f}, 14.2f, 5.38f, run_rs},
+    {F_GEN, 128, 128, 1, 2, 2.96f, 3.61f, 0.00f, 0.91f, {0.746f, 0.751f}, 14.4f, 5.10f, run_gen128},
+    {F_GEN, 256, 128, 1, 1, 0.42f, 6.33f, 0.00f, 1.06f, {0.872f}, 14.0f, 4.85f, run_gen256},
 };
-// whether the form takes the shape (K and the groups in 128-byte stages are the caller's check)
+// Whether the form takes the shape. The ring, split-K and 256 x 256 forms have whole 128-byte stages and 32-bit offsets
+// of codes and outputs, k_gemm_i8g_rs 64-bit offsets of codes; k_gemm_i8g takes everything, and costs less than the
+// others only with several small groups: with one group it is left the shapes that nothing else takes, token tiles of
+// 256 from 512 tokens on.
 static bool form_takes(const GemmForm& f, const GemmArgs& a) {
     if (a.N % f.bn) return false;
+    const bool whole = a.K % 128 == 0 && a.gs % 128 == 0;
+    const bool out32 = (long)a.M * a.ldy < (1L << 30) && (!a.res || (long)a.M * a.ldr < (1L << 30));
+    const bool tiles = whole && out32 && (long)(a.M > a.N ? a.M : a.N) * a.K < (1L << 31);
+    const bool rs = a.M >= 512 && a.K % 256 == 0 && whole && out32;
     switch (f.kind) {
-        case F_W4: return a.M >= 512 && a.K >= 2 * kW4K;
-        case F_RS: return a.M >= 512 && a.K % 256 == 0;
+        case F_W4: return tiles && a.M >= 512 && a.K >= 2 * kW4K;
         // three stages of 384 rows leave room for the scales of 10 groups
-        case F_RING: return f.bm + f.bn < 384 || a.ng <= 10;
-        default: return true;
+        case F_RING: return tiles && (f.bm + f.bn < 384 || a.ng <= 10);
+        case F_SK: return tiles;
+        case F_RS: return rs && (!tiles || a.ng > 1);
+        default: return tiles ? a.ng > 1 : f.bm == 128 ? a.M < 512 : a.M >= 512 && !rs;
     }
 }
 static float form_cost(const GemmForm& f, const GemmArgs& a, int cus) {
     const long nb = (long)(a.N / f.bn) * ((a.M + f.bm - 1) / f.bm), n = (nb + cus - 1) / cus;
-    const float per = (float)(n / f.occ) * f.t[f.occ - 1] + (n % f.occ ? f.t[n % f.occ - 1] : 0.0f);
-    const float stages = (float)(a.K / 128) / f.ks, kb = (float)a.K * 1e-6f;
-    return f.a + fmaxf(stages * per, fmaxf((float)nb * (f.bm + f.bn) * kb / f.bw, (float)a.N * kb / 4.9f));
+    const float stages = (float)(a.K / 128) / f.ks, folds = a.ng > 1 ? (float)a.ng : 0.0f, kb = (float)a.K * 1e-6f;
+    auto T = [&](int r) { return f.e + f.h * r + stages * f.t[r - 1] + folds * f.g * r; };
+    const int rem = (int)(n % f.occ);
+    const float x = (float)(n / f.occ) * T(f.occ) + (rem ? T(rem) : 0.0f), y = (float)nb * (f.bm + f.bn) * kb / f.bw;
+    const float z = (float)a.N * (kb + 4e-6f * a.M) / f.hb;
+    return f.a + sqrtf(x * x + y * y + z * z);
+}
+// The form of a launch: the one that costs least. Q27X_GEMM_W4 = 1 / 0 takes / avoids the 256 x 256 tiles, Q27X_GEMM_FORM
+// = i takes form i of the list, wherever the shape allows (tests of the kernels at small shapes, measurements).
+static const GemmForm* pick_form(const GemmArgs& a, int* index) {
+    const GemmForm* forms = a.ng == 1 ? kFormsK : kFormsG;
+    const int nf = a.ng == 1 ? (int)(sizeof kFormsK / sizeof kFormsK[0]) : (int)(sizeof kFormsG / sizeof kFormsG[0]);
+    const char* ew = getenv("Q27X_GEMM_W4");
+    const char* ef = getenv("Q27X_GEMM_FORM");
+    const bool force = ew && ew[0] == '1' && !ew[1], avoid = ew && ew[0] == '0' && !ew[1];
+    const int want = ef && *ef ? atoi(ef) : -1;
+    const GemmForm* best = nullptr;
+    float cost = 0.0f;
+    for (int i = 0; i < nf; ++i) {
+        const GemmForm& f = forms[i];
+        if (!form_takes(f, a) || (avoid && f.kind == F_W4)) continue;
+        const float c = (i == want || (force && f.kind == F_W4)) ? -1.0f : form_cost(f, a, gemm_cus());
+        if (!best || c < cost) { best = &f; cost = c; *index = i; }
+    }
+    return best;
+}
+static bool gemm_shape_ok(int M, int N, int K, int gs) {
+    return M >= 1 && N >= 1 && K >= 1 && gs >= 1 && !(N % 128) && !(K % kGK) && !(gs % kGK) && !(K % gs) && K / gs <= kGMaxG;
 }
 int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, float alpha, const int8_t* x,
                     const float* sx, int M, void* y, int ldy, int out_bf16, const void* res, int ldr, int res_bf16,
                     float rs, hipStream_t s, const AlphaSel* asel) {
-    if ((N % 128) || (K % kGK) || (gs % kGK) || (K % gs) || K / gs > kGMaxG || ((uintptr_t)w & 15) ||
-        ((uintptr_t)x & 15) || M < 1 || ldy < N || (res && ldr < N)) {
+    if (!gemm_shape_ok(M, N, K, gs) || ((uintptr_t)w & 15) || ((uintptr_t)x & 15) || ldy < N || (res && ldr < N)) {
         set_error("gemm: no kernel for M %d, N %d, K %d, gs %d", M, N, K, gs);
         return Q27X_E_SHAPE;
     }
@@ -1150,46 +1206,22 @@ int launch_gemm_i8g(const int8_t* w, const float* sw, int N, int K, int gs, floa
     a.M = M; a.N = N; a.K = K; a.gs = gs; a.ng = K / gs; a.ldy = ldy; a.ldr = ldr;
     a.out_bf16 = out_bf16; a.res_bf16 = res_bf16;
     if (asel) a.asel = *asel;
-    // Whole 128-byte stages and 32-bit element offsets: the form that costs least. Q27X_GEMM_W4 = 1 / 0 takes /
-    // avoids the 256 x 256 tiles, Q27X_GEMM_FORM = i takes form i of the list, wherever the shape allows (tests of
-    // the kernels at small shapes, measurements).
-    if (K % 128 == 0 && gs % 128 == 0 && (long)(M > N ? M : N) * K < (1L << 31) && (long)M * ldy < (1L << 30) &&
-        (!res || (long)M * ldr < (1L << 30))) {
-        const GemmForm* forms = a.ng == 1 ? kFormsK : kFormsG;
-        const int nf = a.ng == 1 ? (int)(sizeof kFormsK / sizeof kFormsK[0]) : (int)(sizeof kFormsG / sizeof kFormsG[0]);
-        const char* ew = getenv("Q27X_GEMM_W4");
-        const char* ef = getenv("Q27X_GEMM_FORM");
-        const bool force = ew && ew[0] == '1' && !ew[1], avoid = ew && ew[0] == '0' && !ew[1];
-        const int want = ef && *ef ? atoi(ef) : -1;
-        const GemmForm* best = nullptr;
-        float cost = 0.0f;
-        for (int i = 0; i < nf; ++i) {
-            const GemmForm& f = forms[i];
-            if (!form_takes(f, a) || (avoid && f.kind == F_W4)) continue;
-            const float c = (i == want || (force && f.kind == F_W4)) ? -1.0f : form_cost(f, a, gemm_cus());
-            if (!best || c < cost) { best = &f; cost = c; }
-        }
-        if (best) return best->run(a, s);
-    } else if (M >= 512 && K % 256 == 0 && gs % 128 == 0 && (long)M * ldy < (1L << 30) && (!res || (long)M * ldr < (1L << 30))) {
-        return run_rs(a, s);                                         // 2 GiB of codes and more: 64-bit addresses
-    }
-    // other shapes (K or the groups not in 128-byte stages): 64-byte stages, token tiles of 256 (8 waves, one block
-    // per CU, a 5-stage ring) from 512 tokens on, else 128 (4 waves, two blocks per CU, a 4-stage ring, or 3 when 17+
-    // groups' scales take the room)
-    if (M >= 512) {
-        const unsigned mt = (unsigned)((M + 255) / 256);
-        const size_t scl = (size_t)(256 + kGN) * a.ng * sizeof(float);
-        hipLaunchKernelGGL((k_gemm_i8g<256, 5>), dim3((unsigned)(N / kGN) * mt), dim3(512), scl, (hipStream_t)s, a);
-    } else {
-        const unsigned mt = (unsigned)((M + 127) / 128);
-        const size_t scl = (size_t)(128 + kGN) * a.ng * sizeof(float);
-        if (64 * 1024 + scl <= 80 * 1024)
-            hipLaunchKernelGGL((k_gemm_i8g<128, 4>), dim3((unsigned)(N / kGN) * mt), dim3(256), scl, (hipStream_t)s, a);
-        else
-            hipLaunchKernelGGL((k_gemm_i8g<128, 3>), dim3((unsigned)(N / kGN) * mt), dim3(256), scl, (hipStream_t)s, a);
-    }
-    Q27X_HIP(hipGetLastError());
-    return Q27X_OK;
+    int form = 0;
+    return pick_form(a, &form)->run(a, s);     // (a list's general forms take what its others do not)
 }
 
 }  // namespace q27x
+
+extern "C" int q27x_gemm_i8g_form(int M, int N, int K, int gs, int* bm, int* bn) {
+    if (!gemm_shape_ok(M, N, K, gs)) {
+        set_error("q27x_gemm_i8g_form: no kernel for M %d, N %d, K %d, gs %d", M, N, K, gs);
+        return Q27X_E_SHAPE;
+    }
+    GemmArgs a{};
+    a.M = M; a.N = N; a.K = K; a.gs = gs; a.ng = K / gs; a.ldy = N;
+    int form = 0;
+    const GemmForm* f = pick_form(a, &form);
+    if (bm) *bm = f->bm;
+    if (bn) *bn = f->bn;
+    return form;
+}

@@ -2,6 +2,8 @@
 layer-split prefill data path, src/q27_rb.cpp:43-55 and src/q27_epi.hip:14-75, 189-243) against
 the CPU oracle, bit for bit, through the C ABI. The int32 group sums are exact whatever the MFMA
 tiling, and the fp32 slab sum runs in the reference's group order, so outputs match exactly."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -94,29 +96,39 @@ def test_gemm_i8g_wide_tiles(gpu, O, monkeypatch, M, N, K, with_res):
     same(f"wide-tile gemm {M}x{N}x{K}", y, oracle_gemm(O, w, sw, x, sx, K, 0.8125, res, 1.0))
 
 
-# the launch forms in the order of the launcher's lists: (tokens, weight rows) of a tile; (256, 256) and the last
-# grouped form take 512 tokens and more
-FORMS_K = [(16, 32), (32, 32), (32, 32), (32, 64), (64, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256),
-           (256, 128), (256, 256)]
-FORMS_G = [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 128)]
+# the launch forms in the order of the launcher's lists: (tokens, weight rows) of a tile. The (256, 256) tiles and the
+# grouped (256, 128) ones of form 8 take 512 tokens and more.
+FORMS_K = [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 256)]
+FORMS_G = [(16, 32), (32, 32), (32, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 128), (128, 128),
+           (256, 128)]
 
 
-@pytest.mark.parametrize("grouped,form", [(0, i) for i in range(12)] + [(1, i) for i in range(10)])
+def taken(X, M, N, K, gs):
+    bm, bn = ctypes.c_int(), ctypes.c_int()
+    i = X.lib().q27x_gemm_i8g_form(M, N, K, gs, ctypes.byref(bm), ctypes.byref(bn))
+    return i, (bm.value, bn.value)
+
+
+@pytest.mark.parametrize("grouped,form", [(0, i) for i in range(10)] + [(1, i) for i in range(11)])
 def test_gemm_i8g_forms(gpu, O, monkeypatch, grouped, form):
     """Every launch form (Q27X_GEMM_FORM) at the edges of its tiles and K stages: one token, one past a tile,
-    several ragged tiles; one K stage, odd counts, more groups than fit a phase (17 of 1024, 20 of 128)."""
+    several ragged tiles; one K stage, odd counts, more groups than fit a phase (17 of 1024, 20 of 128; the forms whose
+    384 rows leave room for the scales of 10 groups: 10 of 128 and of 512)."""
     monkeypatch.setenv("Q27X_GEMM_FORM", str(form))
     bm, bn = (FORMS_G if grouped else FORMS_K)[form]
     if grouped:
         shapes = [(1, 256, 256, 128), (bm + 1, 512, 2560, 128), (2 * bm + 5, 256, 1152, 384), (37, 256, 17408, 1024)]
-        if form == 9:
+        if form in (6, 7):
+            shapes[1], shapes[3] = (bm + 1, 512, 1280, 128), (37, 256, 5120, 512)
+        if form == 8:
             shapes = [(513, 128, 512, 128), (600, 256, 2560, 128)]
     else:
         shapes = [(1, 256, 128, 128), (bm, 512, 384, 384), (bm + 1, 256, 1152, 1152), (2 * bm + 5, 512, 640, 640),
                   (3, 256, 17408, 17408)]
-        if form == 11:
+        if form == 9:
             shapes = [(512, 256, 256, 256), (769, 512, 1152, 1152)]
     for M, N, K, gs in shapes:
+        assert taken(gpu, M, N, K, gs) == (form, (bm, bn)), (M, N, K, gs)
         rng = np.random.default_rng(0x51E70600 + 100 * form + grouped + M + K)
         ng = K // gs
         w, x = codes(rng, (N, K)), codes(rng, (M, K))
