@@ -625,7 +625,8 @@ __device__ __forceinline__ void tile_rows(AttnArgs& a, int nr, int& pos0, int& n
     a.out += (size_t)r0 * a.nq * HD;
     if (a.xq) { a.xq += (size_t)r0 * a.nq * HD; a.xs += (size_t)r0 * a.nq * HD / 16; }
 }
-template <int HD, int QT>
+// DMA = false: a cache whose codes are not 16-byte aligned (LDS DMA wants that) comes by plain loads and LDS stores.
+template <int HD, int QT, bool DMA>
 __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int nr) {
     warm_args(a);
     if (stopped(a.stop)) return;
@@ -674,14 +675,21 @@ __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int n
             const int u = wv + 8 * i, R = u * kRPI + lane / NCH;
             const int c = (lane % NCH) ^ (R % NCH);
             const size_t off = (size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD + 16 * c;
-            lds_dma16((isv ? a.vc : a.kc) + off,
-                      __builtin_amdgcn_readfirstlane(kv_lds + (uint32_t)(isv * kSplit * HD + 1024 * u)));
+            const int8_t* src = (isv ? a.vc : a.kc) + off;
+            if constexpr (DMA) {
+                lds_dma16(src, __builtin_amdgcn_readfirstlane(kv_lds + (uint32_t)(isv * kSplit * HD + 1024 * u)));
+            } else {
+                uint4 x;
+                __builtin_memcpy(&x, src, 16);
+                *(uint4*)(gdyn + isv * kSplit * HD + 1024 * u + 16 * lane) = x;
+            }
         }
         for (int i = wv; i < (nsc < 8 ? 8 : nsc); i += 8) {          // nsc instructions of 64 scales
             const int j = i & (nsc - 1), f = 64 * j + lane, R = f >> (__builtin_ctz(HD) - gsh), c = f & (nsc - 1);
             const size_t off = (((size_t)(k0 + (R < nk ? R : 0)) * kvrows + (size_t)kvh * HD) >> gsh) + c;
-            lds_dma4((isv ? a.vs : a.ks) + off,
-                     __builtin_amdgcn_readfirstlane(scl_lds + (uint32_t)(isv * kSplit * nsc + 64 * j) * 4u));
+            const float* src = (isv ? a.vs : a.ks) + off;
+            if constexpr (DMA) lds_dma4(src, __builtin_amdgcn_readfirstlane(scl_lds + (uint32_t)(isv * kSplit * nsc + 64 * j) * 4u));
+            else ((float*)(gdyn + 2 * kSplit * HD))[isv * kSplit * nsc + 64 * j + lane] = *src;
         }
     };
     // all but the newest matrix's transfers of this wave have landed
@@ -700,7 +708,8 @@ __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int n
             const int qi = i / (HD / 8), c = i % (HD / 8);
             const int qc = qi < nqr ? qi : 0;                       // rows past nqr: computed, not stored
             const int r = (int)((qc * gdiv) >> 16), g = qc - r * G;
-            const uint4 x = *(const uint4*)(a.qh + (size_t)r * a.nq * HD + (size_t)(kvh * G + g) * HD + 8 * c);
+            uint4 x;                                                // (the caller's rows may start at any element)
+            __builtin_memcpy(&x, a.qh + (size_t)r * a.nq * HD + (size_t)(kvh * G + g) * HD + 8 * c, 16);
             uint32_t* d = sq + qi * QS + c;
             d[0] = __builtin_amdgcn_perm(x.z, x.x, 0x05040100u);
             d[HD / 8] = __builtin_amdgcn_perm(x.z, x.x, 0x07060302u);
@@ -947,13 +956,13 @@ int launch_attn_prep_rows(const AttnArgs& a, int nrows, hipStream_t s) {
     return Q27X_OK;
 }
 
-template <int HD>
+template <int HD, bool DMA>
 static int launch_split_g(const AttnArgs& a, int nr, hipStream_t s) {
     static std::once_flag attr;
     static hipError_t attr_e = hipSuccess;
     std::call_once(attr, [] {
-        const void* f[4] = {(const void*)k_attn_split_g<HD, 1>, (const void*)k_attn_split_g<HD, 2>,
-                            (const void*)k_attn_split_g<HD, 3>, (const void*)k_attn_split_g<HD, 4>};
+        const void* f[4] = {(const void*)k_attn_split_g<HD, 1, DMA>, (const void*)k_attn_split_g<HD, 2, DMA>,
+                            (const void*)k_attn_split_g<HD, 3, DMA>, (const void*)k_attn_split_g<HD, 4, DMA>};
         for (int i = 0; i < 4 && attr_e == hipSuccess; ++i)
             attr_e = hipFuncSetAttribute(f[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_g_lds<HD>(i + 1, HD / 16));
     });
@@ -964,10 +973,10 @@ static int launch_split_g(const AttnArgs& a, int nr, hipStream_t s) {
     const dim3 grid(bx, a.nkv, a.zrows ? (unsigned)((a.ztotal + a.zrows - 1) / a.zrows) : 1u);
     const size_t lds = split_g_lds<HD>(qt, HD / a.kv_group);
     switch (qt) {
-        case 1: hipLaunchKernelGGL((k_attn_split_g<HD, 1>), grid, dim3(kGThreads), lds, s, a, nr); break;
-        case 2: hipLaunchKernelGGL((k_attn_split_g<HD, 2>), grid, dim3(kGThreads), lds, s, a, nr); break;
-        case 3: hipLaunchKernelGGL((k_attn_split_g<HD, 3>), grid, dim3(kGThreads), lds, s, a, nr); break;
-        default: hipLaunchKernelGGL((k_attn_split_g<HD, 4>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        case 1: hipLaunchKernelGGL((k_attn_split_g<HD, 1, DMA>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        case 2: hipLaunchKernelGGL((k_attn_split_g<HD, 2, DMA>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        case 3: hipLaunchKernelGGL((k_attn_split_g<HD, 3, DMA>), grid, dim3(kGThreads), lds, s, a, nr); break;
+        default: hipLaunchKernelGGL((k_attn_split_g<HD, 4, DMA>), grid, dim3(kGThreads), lds, s, a, nr); break;
     }
     Q27X_HIP(hipGetLastError());
     return Q27X_OK;
@@ -1026,7 +1035,9 @@ int launch_attn(const AttnArgs& a, int nr, hipStream_t s, bool prep_fused) {
             if (!a.qh) { set_error("attn: the general geometry needs a query buffer"); return Q27X_E_ARG; }
             if (int rc = launch_attn_prep(a, nr, s)) return rc;
         }
-        const int rc = a.hd == 256 ? launch_split_g<256>(a, nr, s) : launch_split_g<128>(a, nr, s);
+        const bool dma = !(((uintptr_t)a.kc | (uintptr_t)a.vc) & 15);      // (rows are whole 128 bytes)
+        const int rc = a.hd == 256 ? (dma ? launch_split_g<256, true>(a, nr, s) : launch_split_g<256, false>(a, nr, s))
+                                   : (dma ? launch_split_g<128, true>(a, nr, s) : launch_split_g<128, false>(a, nr, s));
         if (rc) return rc;
         if (a.hd == 256) hipLaunchKernelGGL(k_attn_combine<256>, cgrid, dim3(256), comb_lds(a.max_splits, 256), s, a, nr);
         else hipLaunchKernelGGL(k_attn_combine<128>, cgrid, dim3(128), comb_lds(a.max_splits, 128), s, a, nr);

@@ -471,6 +471,39 @@ def test_attention_general_tiles(gpu, O, nq, nkv, hd, group, nr, L0, bad):
     assert np.isfinite(xs_o[:rows]).all()
 
 
+@pytest.mark.parametrize("nq,nkv,hd,group,nr,L0", [
+    (24, 4, 256, 16, 3, 61), (24, 4, 256, 32, 8, 700), (16, 2, 256, 64, 8, 200), (7, 1, 128, 16, 1, 0), (6, 2, 128, 64, 8, 9000)])
+@pytest.mark.parametrize("qoff,coff,soff", [(1, 0, 0), (0, 1, 0), (0, 8, 1), (3, 5, 1)])
+def test_attention_general_any_alignment(gpu, O, nq, nkv, hd, group, nr, L0, qoff, coff, soff):
+    """The general attention kernel on queries, cache codes and scales that start qoff, coff and soff elements past an
+    aligned address, as views into a caller's own buffers do: the bits of the aligned call and of the oracle."""
+    X = gpu
+    rng = np.random.default_rng(L0 + 100 * nr + hd + coff)
+    ctx = L0 + nr
+    kc, ks, vc, vs = fill_kv(rng, O, ctx, nkv, hd, group, ctx)
+    qh = bf16_normal(rng, (nr, nq * hd), 1.0, O=O)
+    gates = bf16_normal(rng, (nr, 2 * nq * hd), 1.0, O=O)
+    out_o = np.empty((nr, nq * hd), np.uint16)
+    xq_o, xs_o = np.empty((nr, nq * hd), np.int8), np.empty((nr, nq * hd // 16), np.float32)
+    O.lib().q27o_attn_rows(qh.ctypes.data, gates.ctypes.data, 2 * nq * hd, kc.ctypes.data, ks.ctypes.data, vc.ctypes.data,
+                           vs.ctypes.data, group, nq, nkv, hd, 1, L0, nr, out_o.ctypes.data, xq_o.ctypes.data,
+                           xs_o.ctypes.data)
+
+    def at(x, off):
+        return dev(X, np.concatenate([np.zeros(off, x.dtype), x.ravel()])), off * x.itemsize
+
+    bufs = [at(qh, qoff), at(gates, 0), at(kc, coff), at(ks, soff), at(vc, coff), at(vs, soff)]
+    pq, pg, pk, pks, pv, pvs = (b.ptr + o for b, o in bufs)
+    work = X.DevBuf(X.lib().q27x_attn_work_bytes(nq, hd, ctx, nr))
+    dout, dxq, dxs = X.DevBuf(nr * nq * hd * 2), X.DevBuf(nr * nq * hd), X.DevBuf(nr * nq * hd // 4)
+    X.call("q27x_attn_rows", pq, pg, 2 * nq * hd, pk, pks, pv, pvs, group, nq, nkv, hd, 1, L0, nr, work.ptr, dout.ptr,
+           dxq.ptr, dxs.ptr, None)
+    X.call("q27x_device_sync")
+    same("attention out", dout.download(np.uint16, (nr, nq * hd)), out_o)
+    same("attention codes", dxq.download(np.int8, (nr, nq * hd)), xq_o)
+    same("attention scales", dxs.download(np.float32, (nr, nq * hd // 16)), xs_o)
+
+
 def test_accept(gpu):
     X = gpu
     for nx, dt, exp in (([5, 6, 7], [5, 6], 2), ([5, 6, 7], [5, 9], 1), ([5, 6, 7], [4, 6], 0), ([1], [], 0)):
