@@ -650,7 +650,7 @@ __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int n
     const float* ksc = (const float*)(gdyn + 2 * kSplit * HD);      // [64][nsc]
     const float* vsc = ksc + kSplit * nsc;
     float* sp = (float*)(gdyn + 2 * kSplit * HD) + 2 * kSplit * nsc;   // [NQ][kSpG] scores, then p
-    __shared__ int sbad;                                            // a V row that some rows do not see is not finite
+    __shared__ int sbad;                                            // a V row that rows multiply by p = 0 may not be finite
     const int t = threadIdx.x, lane = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int g4 = lane >> 4, j16 = lane & 15;
@@ -797,12 +797,14 @@ __global__ __launch_bounds__(kGThreads, 4) void k_attn_split_g(AttnArgs a, int n
         if (more) wait_older();
         else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __syncthreads();
-        // A value that is not finite in a V row that some of the block's rows do not see (p = 0)
-        // would reach them through the matrix cores: such splits take P.V key by key.
-        if (k0 + nk > pos0 + 1) {
+        // A value that is not finite (its scale is not, or a code of up to 128 times it) in a V row that some of the
+        // block's rows do not see (p = 0) would reach them through the matrix cores, and one in the split's first row
+        // would reach all through its copies past the last key: such splits take P.V key by key.
+        if (nk < kSplit || k0 + nk > pos0 + 1) {
             const int kf = pos0 + 1 > k0 ? pos0 + 1 - k0 : 0;       // first key that row 0 does not see
-            for (int i = kf * nsc + t; i < nk * nsc; i += kGThreads)
-                if (!(fabsf(vsc[i]) < __builtin_huge_valf())) sbad = 1;
+            const int ke = nk < kSplit ? nk + 1 : nk;               // ... to the first copy (kf <= nk if there is one)
+            for (int i = kf * nsc + t; i < ke * nsc; i += kGThreads)
+                if (!(fabsf(vsc[i]) * 128.0f < __builtin_huge_valf())) sbad = 1;
         }
         // ---- split softmax as in k_attn_split: four queries of the wave at a time, lane 16 i + c holding
         // keys c, c + 16, c + 32, c + 48 of the pass's i-th; p of key k goes to position

@@ -504,6 +504,38 @@ def test_attention_general_any_alignment(gpu, O, nq, nkv, hd, group, nr, L0, qof
     same("attention scales", dxs.download(np.float32, (nr, nq * hd // 16)), xs_o)
 
 
+@pytest.mark.parametrize("nq,nkv,hd,group", [(24, 4, 256, 32), (24, 4, 256, 16), (6, 2, 128, 64)])
+@pytest.mark.parametrize("nr,L0,key,scale", [
+    (3, 61, 63, 3e38),        # codes times a finite scale overflow in the last key of a full split, which rows 0, 1 do not see
+    (3, 62, 64, 3e38),        # ... in the only key of the next split
+    (4, 130, 133, 2.67e36),   # 127 times this scale is finite, 128 times it is not
+    (2, 70, 64, np.inf),      # an infinite value that every row sees, in the first key of a split that ends early
+    (2, 126, 64, np.inf),     # ... of a full one
+    (1, 0, 0, np.inf)])       # ... the only key
+def test_attention_general_values_that_are_not_finite(gpu, O, nq, nkv, hd, group, nr, L0, key, scale):
+    """V rows whose code x scale is not finite reach the rows that see them, as infinities, and no other row."""
+    X = gpu
+    rng = np.random.default_rng(L0 + 100 * nr + hd)
+    ctx = L0 + nr
+    kc, ks, vc, vs = fill_kv(rng, O, ctx, nkv, hd, group, ctx)
+    vc[key] = np.where(vc[key] == 0, 127, vc[key])               # (a zero code would make a NaN, of no defined bits)
+    vs[key] = scale
+    qh = bf16_normal(rng, (nr, nq * hd), 1.0, O=O)
+    gates = bf16_normal(rng, (nr, 2 * nq * hd), 1.0, O=O)
+    out_o = np.empty((nr, nq * hd), np.uint16)
+    O.lib().q27o_attn_rows(qh.ctypes.data, gates.ctypes.data, 2 * nq * hd, kc.ctypes.data, ks.ctypes.data, vc.ctypes.data,
+                           vs.ctypes.data, group, nq, nkv, hd, 1, L0, nr, out_o.ctypes.data, None, None)
+    dq, dg, dk, dks, dv, dvs = dev(X, qh), dev(X, gates), dev(X, kc), dev(X, ks), dev(X, vc), dev(X, vs)
+    work = X.DevBuf(X.lib().q27x_attn_work_bytes(nq, hd, ctx, nr))
+    dout = X.DevBuf(nr * nq * hd * 2)
+    X.call("q27x_attn_rows", dq.ptr, dg.ptr, 2 * nq * hd, dk.ptr, dks.ptr, dv.ptr, dvs.ptr, group, nq, nkv, hd, 1, L0, nr,
+           work.ptr, dout.ptr, None, None, None)
+    X.call("q27x_device_sync")
+    got = dout.download(np.uint16, (nr, nq * hd))
+    assert not ((out_o & 0x7FFF) > 0x7F80).any()                 # (the oracle's rows hold no NaN)
+    same("attention out", got, out_o)
+
+
 def test_accept(gpu):
     X = gpu
     for nx, dt, exp in (([5, 6, 7], [5, 6], 2), ([5, 6, 7], [5, 9], 1), ([5, 6, 7], [4, 6], 0), ([1], [], 0)):
