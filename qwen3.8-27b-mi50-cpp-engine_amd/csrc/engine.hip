@@ -1428,8 +1428,17 @@ static int pf_streams() {   // chunks in flight: Q27X_PF_STREAMS (1 .. 3), defau
 // columns when they divide K
 static int pf_gs(const q27x_config& c, int K) { return (c.pf_gs > 0 && K % c.pf_gs == 0) ? c.pf_gs : K; }
 
-static int pf_alloc(q27x_ctx* x, int cap, PfBuf** slot) {
-    if (*slot && (*slot)->cap >= cap) return Q27X_OK;
+// Rows that a buffer set for chunks of `rows` rows holds: 512, 1024, 2048 or 4096, at most the context, so that a context
+// whose prompts grow allocates its sets once for each of these and not for each length. (About 300 KB a row of the
+// 5120-wide model: two sets of 2048 rows hold 1.2 GB.)
+static int pf_cap(const q27x_ctx* x, int rows) {
+    int cap = 512;
+    while (cap < rows) cap *= 2;
+    return std::max(rows, std::min(cap, x->c.ctx));
+}
+static int pf_alloc(q27x_ctx* x, int rows, PfBuf** slot) {
+    if (*slot && (*slot)->cap >= rows) return Q27X_OK;
+    const int cap = pf_cap(x, rows);
     if (*slot) {
         Q27X_HIP(hipStreamSynchronize(x->stream));
         for (hipStream_t ps : x->pf_stream) if (ps) Q27X_HIP(hipStreamSynchronize(ps));
@@ -2119,6 +2128,12 @@ int q27x_debug_read(q27x_ctx* x, const char* name, int layer, void* dst, size_t 
         const int32_t cnt = (int32_t)x->pf_walloc.size();
         if (bytes < 4) return Q27X_E_ARG;
         memcpy(dst, &cnt, 4);
+        return Q27X_OK;
+    }
+    if (!strcmp(name, "pf_rows")) {     // rows that the prefill's buffer sets hold
+        const PfBuf* B[3] = {x->pf, x->pfx[0], x->pfx[1]};
+        if (bytes < 12) return Q27X_E_ARG;
+        for (int i = 0; i < 3; ++i) ((int32_t*)dst)[i] = B[i] ? B[i]->cap : 0;
         return Q27X_OK;
     }
     const void* src = nullptr;

@@ -127,6 +127,26 @@ def test_full_width_prefill_wide_gemm_tiles_match_oracle(gpu, O, monkeypatch):
     run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=1024), 520, 2)
 
 
+def test_growing_prompts_keep_their_buffers(gpu):
+    """The prefill's buffer sets come in steps of 512, 1024 and 2048 rows (at most the context): a prompt longer than
+    all before it allocates anew only when its chunks pass a step."""
+    X = gpu
+    cfg = X.tiny_config(spec_k=2, ctx=3000)
+    eng = X.Engine(cfg, SEED)
+    rows = lambda: eng.read("pf_rows", -1, np.int32, 3).tolist()
+    assert rows() == [0, 0, 0]
+    for n, want in ((3, [512, 0, 0]), (300, [512, 0, 0]), (512, [512, 0, 0]), (600, [512, 512, 0]), (900, [512, 512, 0]),
+                    (1024, [512, 512, 0]), (1025, [1024, 1024, 0]), (1300, [1024, 1024, 0]), (2047, [1024, 1024, 0]),
+                    (2400, [2048, 2048, 0]), (2900, [2048, 2048, 0]), (40, [2048, 2048, 0])):
+        eng.prefill_gemm(prompt_of(cfg, n, seed=4))
+        assert rows() == want, n
+    eng.close()
+    eng = X.Engine(X.tiny_config(spec_k=2, ctx=300), SEED)
+    eng.prefill_gemm(prompt_of(cfg, 40, seed=4))
+    assert rows() == [300, 0, 0]
+    eng.close()
+
+
 def test_full_model_spec_equals_plain_after_prefill_gemm(gpu):
     X = gpu
     cfg = X.default_config(spec_k=2, ctx=2048)
