@@ -383,6 +383,8 @@ int q27x_prefill(q27x_ctx* ctx, const int32_t* ids, int n, int32_t* first_token)
  * the decode path's arithmetic; the MTP prompt pass computes only the draft KV cache. Leaves the
  * state fully committed. Its results differ from q27x_prefill's by the quantization granularity. */
 int q27x_prefill_gemm(q27x_ctx* ctx, const int32_t* ids, int n, int32_t* first_token);
+/* Rows per pass over the layers that q27x_prefill_gemm takes for an n-token prompt (no device needed). */
+int q27x_prefill_chunk(int n);
 /* One plain greedy step (Q27_SPEC=0 semantics): consumes the current token, returns the next. */
 int q27x_decode_step(q27x_ctx* ctx, int32_t* out_token);
 /* One chained-MTP speculative round (spec_round, src/q27_main.cpp:2702-2958): K drafts, an

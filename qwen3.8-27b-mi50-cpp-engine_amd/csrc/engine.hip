@@ -1406,16 +1406,21 @@ static int pf_attn_rows(const q27x_config& c, int max_splits, int pos, int left)
     return n;
 }
 static int env_int(const char* name, int def);
-// Rows per pass over the layers for an n-token prompt: up to 512 tokens one chunk, else an even
-// number of equal chunks of at most 2048 rows (whole 64s). Chunks run in pairs on the two streams
-// below, one's GDN scan beside the other's GEMMs: an odd last chunk runs alone, and a short one
-// leaves its partner alone. 16 layers, ms, 512-row chunks below 2048 tokens and 1024-row ones from
+// Rows per pass over the layers for an n-token prompt: up to 512 tokens one chunk, else an even number k of chunks of
+// at most 2048 rows, n / k rounded up to whole 64s (where that would leave fewer than k chunks, to 1); the last chunk
+// takes the rest. Chunks run in pairs on the two streams below, one's GDN scan beside the other's GEMMs: an odd last
+// chunk runs alone, and a short one leaves its partner alone. 16 layers, ms, 512-row chunks below 2048 tokens and 1024-row ones from
 // there / now: 600 tokens 11.6 / 11.0, 1300 21.9 / 18.3, 2600 40.0 / 37.1, 3300 51.8 / 49.5, 5000
 // 82.7 / 78.4, 8000 147.4 / 144.2; 300 tokens in two chunks 2.6 against 2.2 (4 layers).
 // Q27X_PF_CHUNK (8 .. 4096) overrides, read per call.
 static int pf_chunk(int n) {
-    const int k = n <= 512 ? 1 : 2 * ((n + 4095) / 4096);
-    const int v = env_int("Q27X_PF_CHUNK", n <= 512 ? 512 : ((n + k - 1) / k + 63) / 64 * 64);
+    int rows = 512;
+    if (n > 512) {
+        const int k = 2 * ((n - 1) / 4096 + 1), even = (n - 1) / k + 1;
+        rows = (even + 63) / 64 * 64;
+        if ((n - 1) / rows + 1 < k) rows = even;
+    }
+    const int v = env_int("Q27X_PF_CHUNK", rows);
     return v < 8 ? 8 : (v > 4096 ? 4096 : v);
 }
 // successive chunks on two streams, chunk c + 1's layer l behind chunk c's layer l (Q27X_PF_PIPE=0: one
@@ -1623,6 +1628,11 @@ static int pf_mtp(q27x_ctx* x, int p0, int C) {
     a.nq = c.n_q; a.nkv = c.n_kv; a.hd = c.head_dim; a.gate = c.attn_gate; a.eps = c.rms_eps;
     a.pos0_imm = p0; a.prep_kv_only = 1; a.stop = &d->stop;
     return launch_attn_prep_rows(a, C, x->pfs);
+}
+
+int q27x_prefill_chunk(int n) {
+    if (n < 1) { set_error("q27x_prefill_chunk: %d tokens", n); return Q27X_E_ARG; }
+    return pf_chunk(n);
 }
 
 int q27x_prefill_gemm(q27x_ctx* x, const int32_t* ids, int n, int32_t* first_token) {

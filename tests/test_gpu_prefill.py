@@ -62,7 +62,7 @@ def run_case(X, O, cfg, n, rounds, chunk=None, seed=3):
         om.close()
 
 
-@pytest.mark.parametrize("n,chunk,gs", [(1, None, 0), (9, None, 0), (300, None, 0), (150, 64, 0), (70, 8, 0),
+@pytest.mark.parametrize("n,chunk,gs", [(1, None, 0), (9, None, 0), (300, None, 0), (150, 64, 0), (150, 37, 0), (70, 8, 0),
                                         (300, None, 1024), (70, 8, 1024)])
 def test_tiny_prefill_gemm_matches_oracle(gpu, O, n, chunk, gs):
     """gs: the K-group of the trunk's GEMMs (Q27_Q8_GS): 0 = the whole K (the reference default),
