@@ -170,7 +170,7 @@ def test_bf16_gemv(gpu, O, nr):
 @pytest.mark.parametrize("n,off", [(1, 0), (3, 0), (4, 0), (4099, 0), (62080, 0), (40001, 1)])
 def test_argmax_rows_edges(gpu, O, n, off):
     """Ties across threads and waves, zeros of both signs, rows without a finite value, widths with a remainder and
-    rows that 16-byte loads cannot take."""
+    rows that start at any element."""
     X = gpu
     rng = np.random.default_rng(n)
     y = rng.integers(-3, 4, (4, n)).astype(np.float32)                # many ties

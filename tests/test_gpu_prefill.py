@@ -3,8 +3,9 @@ restatement (q27o_model_prefill_gemm): after the prompt, the first token and the
 state bit for bit (h_prev, every GDN layer's state and conv history, every attention layer's and
 the MTP layer's KV cache), then speculative rounds continuing from it, round by round with their
 drafts and hand-off. Prompts span several chunks (Q27X_PF_CHUNK) and several attention launches
-(128 query rows each); the the model's widths run at 4 layers; the full 64-layer model checks that
+(128 query rows each); the model's widths run at 4 layers; the full 64-layer model checks that
 spec == plain greedy after a GEMM prefill."""
+import ctypes
 import os
 
 import numpy as np
@@ -118,13 +119,30 @@ def test_full_width_prefill_gemm_matches_oracle(gpu, O, n, chunk, gs):
     run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=512, pf_gs=gs), n, 2, chunk)
 
 
+# (weight rows, K) of the prefill's GEMMs at the model's widths: in_qkv|in_z, out_proj, q|k|v, o, gate|up, down, the MTP fc
+WIDE = [(16384, 5120), (5120, 6144), (10240, 5120), (5120, 4096), (34816, 5120), (5120, 17408), (5120, 5120)]
+
+
 def test_full_width_prefill_wide_gemm_tiles_match_oracle(gpu, O, monkeypatch):
     """The 256 x 256 GEMM tiles in every epilogue form the prefill uses (fp32 and bf16 outputs, the
     bf16 residual of down, out_proj and o_proj) at the model's widths: 520 tokens in a 512-row
     chunk (the tiles need 512 rows) and an 8-row one, with the tiles forced wherever the shape
     allows them (Q27X_GEMM_W4 = 1); state after the prompt and two rounds bit for bit."""
     monkeypatch.setenv("Q27X_GEMM_W4", "1")
-    run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=1024), 520, 2)
+    for N, K in WIDE:
+        bm, bn = ctypes.c_int(), ctypes.c_int()
+        assert gpu.lib().q27x_gemm_i8g_form(512, N, K, K, ctypes.byref(bm), ctypes.byref(bn)) >= 0
+        assert (bm.value, bn.value) == (256, 256), (N, K)
+    run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=1024), 520, 2, 512)
+
+
+def test_full_width_prefill_grouped_wide_gemm_tiles_match_oracle(gpu, O, monkeypatch):
+    """The same for the register-staged 256 x 128 tiles, with 1024-column groups (Q27X_GEMM_FORM = 8 of the grouped
+    list; the MTP's whole-K GEMMs take form 8 of theirs, 256 x 128 ring tiles)."""
+    monkeypatch.setenv("Q27X_GEMM_FORM", "8")
+    for N, K in WIDE[:-1]:
+        assert gpu.lib().q27x_gemm_i8g_form(512, N, K, 1024, None, None) == 8, (N, K)
+    run_case(gpu, O, gpu.default_config(spec_k=2, n_layers=4, ctx=1024, pf_gs=1024), 520, 2, 512)
 
 
 def test_growing_prompts_keep_their_buffers(gpu):

@@ -49,20 +49,27 @@ def oracle_gemm(O, w, sw, x, sx, gs, alpha, res=None, rs=0.0):
     return y
 
 
+def taken(X, M, N, K, gs):
+    bm, bn = ctypes.c_int(), ctypes.c_int()
+    i = X.lib().q27x_gemm_i8g_form(M, N, K, gs, ctypes.byref(bm), ctypes.byref(bn))
+    return i, (bm.value, bn.value)
+
+
+# shapes that few weight rows send to split-K tiles, whatever the tokens; the other forms are below
 @pytest.mark.parametrize("M,N,K,gs,with_res", [
     (1, 128, 1024, 1024, False),       # one token, one group
-    (37, 256, 5120, 1024, True),       # ragged token tile, residual
-    (128, 128, 2048, 1024, False),     # exactly one tile
+    (37, 256, 5120, 1024, True),       # ragged token tiles, residual
+    (128, 128, 2048, 1024, False),     # whole token tiles
     (300, 384, 5120, 5120, True),      # one group over the whole K (per-token scales)
     (130, 256, 17408, 1024, False),    # down's K: 17 groups
     (257, 128, 6144, 1024, True),      # out_proj's K
-    (600, 256, 5120, 1024, True),      # 256-token tiles (register-staged), ragged last tile
-    (1024, 384, 17408, 1024, False),   # 256-token tiles (register-staged), 17 groups
-    (520, 128, 1152, 1152, True),      # 256-token tiles, K % 256 != 0: the LDS-DMA ring
-    (777, 256, 3200, 640, False),      # 256-token tiles, K % 256 != 0, 5 groups of 640
-    (600, 256, 5120, 5120, True),      # 256-token tiles, one group over the whole K (the default arm)
+    (600, 256, 5120, 1024, True),      # 32 x 32 tiles, a ragged last one
+    (1024, 384, 17408, 1024, False),   # 32 x 64 tiles, 17 groups
+    (520, 128, 1152, 1152, True),      # an odd number of K stages
+    (777, 256, 3200, 640, False),      # 5 groups of 640
+    (600, 256, 5120, 5120, True),      # 32 x 32 tiles, one group over the whole K (the default arm)
     (130, 256, 17408, 17408, False),   # down's K as one group
-    (1024, 384, 17408, 17408, True),   # 256-token tiles, down's K as one group
+    (1024, 384, 17408, 17408, True),   # 32 x 64 tiles, down's K as one group
 ])
 def test_gemm_i8g(gpu, O, M, N, K, gs, with_res):
     rng = np.random.default_rng(0x51E70400 + M + N + K)
@@ -76,6 +83,31 @@ def test_gemm_i8g(gpu, O, M, N, K, gs, with_res):
     same(f"gemm {M}x{N}x{K}/{gs}", y, oracle_gemm(O, w, sw, x, sx, gs, 0.8125, res, 1.0))
 
 
+@pytest.mark.parametrize("M,N,K,gs,with_res,tile", [
+    (1, 128, 64, 64, False, (128, 128)),         # one K stage of 64 bytes
+    (77, 256, 1088, 1088, True, (128, 128)),     # one group, an odd number of stages, a ragged tile
+    (300, 256, 1088, 64, True, (128, 128)),      # 17 groups: the 3-stage ring
+    (511, 128, 1280, 64, False, (128, 128)),     # 20 groups
+    (130, 384, 1152, 192, True, (128, 128)),     # groups of three half stages
+    (512, 128, 64, 64, True, (256, 128)),        # 256-token tiles: one stage
+    (600, 256, 1088, 1088, False, (256, 128)),   # a ragged last tile, one group
+    (777, 256, 1152, 192, True, (256, 128)),
+    (1025, 128, 3200, 320, False, (256, 128)),   # 10 groups
+    (600, 384, 1280, 64, True, (256, 128)),      # 20 groups
+])
+def test_gemm_i8g_half_stages(gpu, O, M, N, K, gs, with_res, tile):
+    """K or groups with half a 128-byte stage left over: the general kernel's 64-byte stages."""
+    assert taken(gpu, M, N, K, gs)[1] == tile
+    rng = np.random.default_rng(0x51E70700 + M + N + K + gs)
+    w, x = codes(rng, (N, K)), codes(rng, (M, K))
+    w[0], x[0] = 127, -127
+    sw = rng.uniform(1e-4, 2e-3, (N, K // gs)).astype(np.float32)
+    sx = rng.uniform(1e-3, 5e-2, (M, K // gs)).astype(np.float32)
+    res = rng.standard_normal((M, N)).astype(np.float32) if with_res else None
+    y = gpu_gemm(gpu, w, sw, x, sx, gs, 0.8125, res, 1.0)
+    same(f"half-stage gemm {M}x{N}x{K}/{gs}", y, oracle_gemm(O, w, sw, x, sx, gs, 0.8125, res, 1.0))
+
+
 @pytest.mark.parametrize("M,N,K,with_res", [
     (512, 256, 256, False),     # one tile, two K stages
     (600, 512, 5120, True),     # ragged last token tile, two weight tiles, residual
@@ -84,8 +116,9 @@ def test_gemm_i8g(gpu, O, M, N, K, gs, with_res):
 ])
 def test_gemm_i8g_wide_tiles(gpu, O, monkeypatch, M, N, K, with_res):
     # the 256 x 256 tiles of the whole-K arm, taken at shapes where the launch would otherwise use
-    # the 256 x 128 ones (Q27X_GEMM_W4 = 1), against the oracle bit for bit
+    # smaller ones (Q27X_GEMM_W4 = 1), against the oracle bit for bit
     monkeypatch.setenv("Q27X_GEMM_W4", "1")
+    assert taken(gpu, M, N, K, K)[1] == (256, 256)
     rng = np.random.default_rng(0x51E70500 + M + N + K)
     w, x = codes(rng, (N, K)), codes(rng, (M, K))
     w[0], x[0] = 127, -127
@@ -101,12 +134,6 @@ def test_gemm_i8g_wide_tiles(gpu, O, monkeypatch, M, N, K, with_res):
 FORMS_K = [(16, 32), (32, 32), (32, 64), (64, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 256)]
 FORMS_G = [(16, 32), (32, 32), (32, 64), (64, 128), (64, 256), (128, 128), (128, 256), (256, 128), (256, 128), (128, 128),
            (256, 128)]
-
-
-def taken(X, M, N, K, gs):
-    bm, bn = ctypes.c_int(), ctypes.c_int()
-    i = X.lib().q27x_gemm_i8g_form(M, N, K, gs, ctypes.byref(bm), ctypes.byref(bn))
-    return i, (bm.value, bn.value)
 
 
 @pytest.mark.parametrize("grouped,form", [(0, i) for i in range(10)] + [(1, i) for i in range(11)])
