@@ -597,7 +597,11 @@ __global__ __launch_bounds__(HD) void k_attn_combine(AttnArgs a, int nr) {
 //     same work at any QT. The second half's waves add c2, then c3 to the first's c0 + c1 in LDS.
 //   P.V: wave w owns HD/128 16-dim tiles for all query tiles.
 // At most 128 registers and half of a CU's LDS, so two blocks share a CU and one's softmax and waits
-// are covered by the other's matrix work.
+// are covered by the other's matrix work. (256 dims with 4 query tiles, a prefill's row tiles in GQA
+// groups of 4 and more, are short of registers: 28 bytes of scratch per lane, reloaded between the request
+// of the next K and the wait for V. They count as newer, so that wait takes in the next K as well: right,
+// but without the overlap.) 24q/4kv x 256, 8 rows at 16003 positions: 51 us; matrix instructions take 45%
+// of the SIMDs' cycles, the other vector instructions (operands widened, softmax) 43%.
 constexpr int kGThreads = 512;
 // x, as a value the compiler cannot move out of the loop it is taken in
 __device__ __forceinline__ int opaque(int x) {

@@ -21,8 +21,8 @@
 // x 64 to 256 weight rows per block, 128-byte K stages in an LDS ring), k_gemm_i8g_sk (few tokens: small tiles whose
 // waves split K), k_gemm_i8g_w4 (256 x 256 tiles, one group over K) and k_gemm_i8g_rs (256 x 128, several groups). At
 // the end of each group the int32 tiles are folded into fp32 accumulators with the group's scales and restarted
-// from zero. The general form for the other shapes, k_gemm_i8g: a 256-thread block computes a 128-token x 128-row
-// tile; wave w owns the 64 x 64 quarter (w / 2, w % 2) as 2 x 2 v_mfma_i32_32x32x32_i8 tiles, and two blocks share a
+// from zero. The general form, k_gemm_i8g, takes the other shapes and some with several small groups: a 256-thread
+// block computes a 128-token x 128-row tile; wave w owns the 64 x 64 quarter (w / 2, w % 2) as 2 x 2 v_mfma_i32_32x32x32_i8 tiles, and two blocks share a
 // CU. K advances 64 bytes per stage through a ring of 4 LDS stages (3 when the scales of 17+ groups take the room)
 // filled by LDS DMA ahead of the multiply.
 #include <math.h>
@@ -868,8 +868,9 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_i8g_sk(GemmArgs a, int gpp) {
 
 // Weights: per-64 mirror -> per-(row, group) codes and scales; one wave per (row, group). In place when wg == w (each
 // element is read and written by the same thread). Bound by memory: 16 codes per lane and load, four loads in flight
-// (a byte per lane and load: 16384 x 5120 96 us, now 34: 4.9 TB/s). VEC = 0 is the byte form, for codes that are not 16-byte
-// aligned.
+// (a byte per lane and load: 16384 x 5120 96 us, now 34: 4.9 TB/s). A pass is 4096 codes whatever the group, so with
+// narrower groups lanes load and convert codes that they do not store: on cached codes, in groups of 5120 68 us and now
+// 28, of 1024 87 / 31, of 256 155 / 104, of 64 494 / 408. VEC = 0 is the byte form, for codes that are not 16-byte aligned.
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_i8g64_to_grp(const int8_t* w, const float* s64, int rows, int K, int gs,
                                                       int8_t* wg, float* sg) {
