@@ -2,8 +2,8 @@
 restatement (q27o_model_prefill_gemm): after the prompt, the first token and the whole committed
 state bit for bit (h_prev, every GDN layer's state and conv history, every attention layer's and
 the MTP layer's KV cache), then speculative rounds continuing from it, round by round with their
-drafts and hand-off. Prompts span several chunks (Q27X_PF_CHUNK) and several attention launches
-(128 query rows each); the model's widths run at 4 layers; the full 64-layer model checks that
+drafts and hand-off. Prompts span several chunks (Q27X_PF_CHUNK) and, near the end of the
+context, several attention launches (300 of 512 positions: 256 and 44 query rows); the model's widths run at 4 layers; the full 64-layer model checks that
 spec == plain greedy after a GEMM prefill."""
 import ctypes
 import os
